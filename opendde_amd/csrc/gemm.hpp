@@ -58,7 +58,8 @@ struct GemmShape {
   static constexpr int OPS_A = TX / RPO / 8, OPS_B = TY / RPO / 8;  // 1 KiB loads per wave
   static constexpr int OPS = OPS_A + OPS_B;
   static constexpr int STAGE_ELEMS = (TX + TY) * KC;          // bf16 per stage
-  static_assert(TX % (16 * 8) == 0 && TY % (16 * 8) == 0, "16-row blocks per wave");
+  static_assert(TX % (16 * WX) == 0 && TY % (16 * WY) == 0, "16-row blocks per wave");
+  static_assert(TX % (8 * RPO) == 0 && TY % (8 * RPO) == 0, "whole loads per wave");
 };
 
 // arow(r) / brow(r): pointer to element k = 0 of the tile's A row r
@@ -258,13 +259,17 @@ __device__ __forceinline__ void gemm_nt_mainloop_pipe64_k(
           mma(acc[i][j], fa[set][i], fb[set][j]);
         }
       }
-    // one LDS read after each MFMA pair (reads requested just before)
+    // one LDS read after each MFMA pair (reads requested just before), or
+    // after each MFMA where a small wave block has fewer than two per read
+    constexpr int PER = MX * MY >= 2 * (MX + MY) ? 2 : 1;
+    static_assert(MX * MY >= MX + MY, "an MFMA for every read");
 #pragma unroll
     for (int k = 0; k < MX + MY; ++k) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+      __builtin_amdgcn_sched_group_barrier(0x008, PER, 0);
       __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
     }
-    __builtin_amdgcn_sched_group_barrier(0x008, MX * MY - 2 * (MX + MY), 0);
+    if constexpr (MX * MY > PER * (MX + MY))
+      __builtin_amdgcn_sched_group_barrier(0x008, MX * MY - PER * (MX + MY), 0);
   };
   using I0 = std::integral_constant<int, 0>;
   using I1 = std::integral_constant<int, 1>;

@@ -8,7 +8,7 @@
 //                        Incoming reads z through swapped strides, which
 //                        writes a[k,i] at A[c][i][k]: no transposed copy.
 //   2. trimul_contract — P[c][x][y] = sum_k A[c][x][k] B[c][y][k]: a batched
-//                        NT GEMM on MFMA, 128x128 tiles, LDS-staged K blocks,
+//                        NT GEMM on MFMA, LDS-staged K blocks,
 //                        XCD-aware tile order (all tiles of one channel on
 //                        one XCD so A_c and B_c stay in that XCD's L2).
 //   3. trimul_out      — per pair row: LN_out over the channel-major P
@@ -16,8 +16,10 @@
 //                        sigmoid(W_g LN_in(z)) recomputed from z (which is
 //                        read for the residual anyway), plus the residual.
 //
-// Workspace (CT = compute type, Np = N rounded up to 128):
-//   A, B, P : [Ch][Np][Np]
+// Workspace (CT = compute type, Np = N rounded up to 64, or to 256 for the
+// three-part contraction):
+//   A, B, P : [Ch][Np][Np]; rows x >= N of A and B are not written, and rows
+//   and columns of P past N hold no value (they are read, never used)
 #include <string.h>
 
 #include "common.hpp"
@@ -212,25 +214,11 @@ struct ContractArgs {
   int np, ch;
 };
 
-template <typename CT> struct ContractCfg;
-template <> struct ContractCfg<bf16> { static constexpr int BK = 64; static constexpr int PAD = 8; };
-template <> struct ContractCfg<float> { static constexpr int BK = 32; static constexpr int PAD = 4; };
-
-template <typename CT>
-__global__ __launch_bounds__(256) void trimul_contract_kernel(ContractArgs<CT> a) {
-  constexpr int BK = ContractCfg<CT>::BK;
-  constexpr int LD = BK + ContractCfg<CT>::PAD;
-  constexpr int VEC = 16 / sizeof(CT);            // elements per 16-byte chunk
-  constexpr int CHUNKS = 128 * BK / VEC;          // chunks per operand tile
-  __shared__ __attribute__((aligned(16))) CT As[128 * LD];
-  __shared__ __attribute__((aligned(16))) CT Bs[128 * LD];
-
-  const int T = a.np / 128;
-  const int tiles = T * T;
-  // XCD-aware order: workgroup ids are dealt round-robin over 8 XCDs; give
-  // every tile of one channel to the same XCD when the channel count allows.
-  int bid = blockIdx.x, c, tile;
-  if ((a.ch & 7) == 0) {
+// blockIdx -> (channel, tile): workgroup ids are dealt round-robin over 8
+// XCDs; every tile of one channel goes to the same XCD when the channel count
+// allows.
+__device__ __forceinline__ void contract_tile_map(int bid, int ch, int tiles, int& c, int& tile) {
+  if ((ch & 7) == 0) {
     const int xcd = bid & 7, local = bid >> 3;
     c = (local / tiles) * 8 + xcd;
     tile = local % tiles;
@@ -238,75 +226,112 @@ __global__ __launch_bounds__(256) void trimul_contract_kernel(ContractArgs<CT> a
     c = bid / tiles;
     tile = bid % tiles;
   }
-  const int x0 = (tile / T) * 128, y0 = (tile % T) * 128;
+}
+
+// fp32 form: T x T tiles (Np a multiple of T) per workgroup of 4 waves, each
+// T/2 x T/2, bound by the fp32 MFMA.  K blocks are double-buffered in LDS:
+// block k + 2 waits in registers while block k is multiplied, one barrier per
+// block (N = 512: 116 TF/s; a large fp32 matrix product reaches 154).
+template <int T>
+__global__ __launch_bounds__(256) void trimul_contract_f32_kernel(ContractArgs<float> a) {
+  constexpr int BK = 32;
+  constexpr int LD = BK + 4;
+  constexpr int VEC = 4;                          // elements per 16-byte chunk
+  constexpr int CPR = BK / VEC;                   // chunks per row
+  constexpr int PPT = T * CPR / 256;              // chunks per thread and operand
+  constexpr int M = T / 32;                       // fragments per wave and operand
+  static_assert(T * CPR % 256 == 0, "whole chunks per thread");
+  __shared__ __attribute__((aligned(16))) float As[2][T * LD];
+  __shared__ __attribute__((aligned(16))) float Bs[2][T * LD];
+
+  const int Tn = a.np / T;
+  int c, tile;
+  contract_tile_map(blockIdx.x, a.ch, Tn * Tn, c, tile);
+  const int x0 = (tile / Tn) * T, y0 = (tile % Tn) * T;
   const int w = wave_id(), l = lane_id(), g = l >> 4, r16 = l & 15;
   const int wm = w >> 1, wn = w & 1;
   const size_t plane = (size_t)a.np * a.np;
-  const CT* Ab = a.A + c * plane + (size_t)x0 * a.np;
-  const CT* Bb = a.B + c * plane + (size_t)y0 * a.np;
+  const float* Ab = a.A + c * plane + (size_t)x0 * a.np;
+  const float* Bb = a.B + c * plane + (size_t)y0 * a.np;
 
-  f32x4 acc[4][4];
+  f32x4 acc[M][M];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
-    for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int i = 0; i < M; ++i)
+    for (int j = 0; j < M; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  for (int k0 = 0; k0 < a.np; k0 += BK) {
+  f32x4 ra[PPT], rb[PPT];
+  auto load = [&](int k0) {
 #pragma unroll
-    for (int it = 0; it < CHUNKS / 256; ++it) {
+    for (int it = 0; it < PPT; ++it) {
       const int ci = threadIdx.x + it * 256;
-      const int r = ci / (BK / VEC), cc = (ci % (BK / VEC)) * VEC;
-      *reinterpret_cast<f32x4*>(&As[r * LD + cc]) =
-          *reinterpret_cast<const f32x4*>(Ab + (size_t)r * a.np + k0 + cc);
-      *reinterpret_cast<f32x4*>(&Bs[r * LD + cc]) =
-          *reinterpret_cast<const f32x4*>(Bb + (size_t)r * a.np + k0 + cc);
+      const int r = ci / CPR, cc = (ci % CPR) * VEC;
+      ra[it] = *reinterpret_cast<const f32x4*>(Ab + (size_t)r * a.np + k0 + cc);
+      rb[it] = *reinterpret_cast<const f32x4*>(Bb + (size_t)r * a.np + k0 + cc);
     }
-    __syncthreads();
+  };
+  auto stage = [&](int buf) {
+#pragma unroll
+    for (int it = 0; it < PPT; ++it) {
+      const int ci = threadIdx.x + it * 256;
+      const int r = ci / CPR, cc = (ci % CPR) * VEC;
+      *reinterpret_cast<f32x4*>(&As[buf][r * LD + cc]) = ra[it];
+      *reinterpret_cast<f32x4*>(&Bs[buf][r * LD + cc]) = rb[it];
+    }
+  };
+  const int nst = a.np / BK;
+  load(0);
+  stage(0);
+  if (nst > 1) load(BK);
+  lds_barrier();
+  for (int st = 0; st < nst; ++st) {
+    const float* as = As[st & 1];
+    const float* bs = Bs[st & 1];
 #pragma unroll
     for (int kk = 0; kk < BK; kk += 32) {
-      Frag<CT> af[4], bfr[4];
+      Frag<float> af[M], bfr[M];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        af[i].load(&As[(wm * 64 + i * 16 + r16) * LD + kk + 8 * g]);
-        bfr[i].load(&Bs[(wn * 64 + i * 16 + r16) * LD + kk + 8 * g]);
+      for (int i = 0; i < M; ++i) {
+        af[i].load(&as[(wm * (T / 2) + i * 16 + r16) * LD + kk + 8 * g]);
+        bfr[i].load(&bs[(wn * (T / 2) + i * 16 + r16) * LD + kk + 8 * g]);
       }
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int i = 0; i < M; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) mma(acc[i][j], bfr[j], af[i]);
+        for (int j = 0; j < M; ++j) mma(acc[i][j], bfr[j], af[i]);
     }
-    __syncthreads();
+    // the other buffer was last read in block st - 1, before the barrier
+    // that ended it
+    if (st + 1 < nst) {
+      stage((st + 1) & 1);
+      if (st + 2 < nst) load((st + 2) * BK);
+      lds_barrier();
+    }
   }
-  // acc[i][j]: column = row x (x0 + 64wm + 16i + r16), rows y = y0 + 64wn + 16j + 4g + r
-  CT* Pb = a.P + c * plane;
+  // acc[i][j]: column = row x (x0 + T/2 wm + 16i + r16), rows y = y0 + T/2 wn + 16j + 4g + r
+  float* Pb = a.P + c * plane;
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < M; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int xx = x0 + wm * 64 + i * 16 + r16;
-      const int yy = y0 + wn * 64 + j * 16 + 4 * g;
+    for (int j = 0; j < M; ++j) {
+      const int xx = x0 + wm * (T / 2) + i * 16 + r16;
+      const int yy = y0 + wn * (T / 2) + j * 16 + 4 * g;
       store4(Pb + (size_t)xx * a.np + yy, acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]);
     }
 }
 
-// Large-tile form (bf16, Np a multiple of 256): TX x TY tiles per workgroup
-// of 8 waves, the shared NT mainloop (gemm.hpp) over k = 0..Np.
+// Large-tile form (bf16): TX x TY tiles per workgroup of 8 waves, the shared
+// NT mainloop (gemm.hpp) over k = 0..Np.  The last tile of a dimension may
+// reach past Np: its rows there repeat row Np - 1 and are not stored.
 template <int TX, int TY, int WX, int NS, int KC, bool kPipe = false>
 __global__ __launch_bounds__(512) void trimul_contract_big_kernel(ContractArgs<bf16> a) {
   using S = GemmShape<TX, TY, WX, KC>;
   static_assert(!kPipe || (KC == 64 && NS == 2), "the pipelined mainloop: two 64-k stages");
   __shared__ __attribute__((aligned(16))) bf16 sm[NS * S::STAGE_ELEMS];
-  const int TXn = a.np / TX, TYn = a.np / TY;
-  const int tiles = TXn * TYn;
-  int bid = blockIdx.x, c, tile;
-  if ((a.ch & 7) == 0) {  // all tiles of a channel on one XCD
-    const int xcd = bid & 7, local = bid >> 3;
-    c = (local / tiles) * 8 + xcd;
-    tile = local % tiles;
-  } else {
-    c = bid / tiles;
-    tile = bid % tiles;
-  }
+  const int TXn = (a.np + TX - 1) / TX, TYn = (a.np + TY - 1) / TY;
+  int c, tile;
+  contract_tile_map(blockIdx.x, a.ch, TXn * TYn, c, tile);
   const int x0 = (tile / TYn) * TX, y0 = (tile % TYn) * TY;
+  const int xr = min(TX, a.np - x0), yr = min(TY, a.np - y0);  // rows inside Np
   const size_t plane = (size_t)a.np * a.np;
   f32x4 acc[S::MX][S::MY];
   const bf16* Ab = a.A + c * plane + (size_t)x0 * a.np;
@@ -315,18 +340,19 @@ __global__ __launch_bounds__(512) void trimul_contract_big_kernel(ContractArgs<b
   // each 32 rows, row block 2p + b, MFMA row m is column 8 (m >> 2) + 4 b +
   // (m & 3), so a lane's results of row blocks 2p and 2p + 1 are 8
   // consecutive columns (one 16-byte store)
-  auto arow = [&](int r) { return Ab + (size_t)r * a.np; };
+  auto arow = [&](int r) { return Ab + (size_t)min(r, xr - 1) * a.np; };
   auto brow = [&](int r) {
     const int m = r & 15;
-    return Bb + (size_t)((r & ~31) + 8 * (m >> 2) + 4 * ((r >> 4) & 1) + (m & 3)) * a.np;
+    return Bb +
+           (size_t)min((r & ~31) + 8 * (m >> 2) + 4 * ((r >> 4) & 1) + (m & 3), yr - 1) * a.np;
   };
   if constexpr (kPipe) {
     // buffer-resource loads based at the tile's first A and B rows
     GemmBufs bufs;
     bufs.a = Ab;
-    bufs.a_bytes = (uint32_t)((size_t)TX * a.np * sizeof(bf16));
+    bufs.a_bytes = (uint32_t)((size_t)xr * a.np * sizeof(bf16));
     bufs.b = Bb;
-    bufs.b_bytes = (uint32_t)((size_t)TY * a.np * sizeof(bf16));
+    bufs.b_bytes = (uint32_t)((size_t)yr * a.np * sizeof(bf16));
     gemm_nt_mainloop_pipe64_k<TX, TY, WX, true, true>(
         arow, brow, a.np / 64, [](bool, int st) { return st * 64; }, sm, acc, bufs);
   } else
@@ -347,6 +373,8 @@ __global__ __launch_bounds__(512) void trimul_contract_big_kernel(ContractArgs<b
     for (int j = 0; j < S::MY; j += 4) {
       const int xx = x0 + wx * (TX / WX) + i * 16 + r16;
       const int y = y0 + wy * (TY / S::WY) + j * 16;
+      if (y >= a.np) continue;  // Np is a multiple of the line's 64 columns
+      const bool ok = xx < a.np;  // and of the pair's two rows
       bf16x8 lo, hi;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
@@ -356,41 +384,85 @@ __global__ __launch_bounds__(512) void trimul_contract_big_kernel(ContractArgs<b
         hi[4 + e] = (bf16)acc[i][j + 3][e];
       }
       store_line_pair(reinterpret_cast<bf16x8*>(Pb + (size_t)xx * a.np + y),
-                      reinterpret_cast<bf16x8*>(Pb + (size_t)(xx ^ 1) * a.np + y), g, lo, hi);
+                      reinterpret_cast<bf16x8*>(Pb + (size_t)(xx ^ 1) * a.np + y), g, lo, hi, ok,
+                      ok);
     }
 }
 
-// Np >= 768: 256 x 256 tiles staged 64 k at a time (whole 128-byte lines of
-// each row; 128 KiB of LDS, one workgroup per CU), software-pipelined, each
-// wave a 64 x 128 block; Np = 512: 256 x 128 tiles staged 32 k at a time
-// (two workgroups per CU), which keeps more workgroups per channel.  Chosen
-// by measurement on MI355X (N = 1024: the pipelined loop 0.311 / 0.281 ms
-// outgoing / incoming against 0.317 / 0.290 ms for the plain one; deeper
-// 32-k staging, with or without a k-blocked operand layout, was slower;
-// N = 768: 0.138 against 0.152 ms for the 256 x 128 form).
-// ODDE_CONTRACT_TILE=256x256 or 256x128 overrides the choice by Np (tuning).
+// Tile of the bf16 contraction.  The mainloop of every large tile is the
+// software-pipelined one (whole 128-byte lines, 64 k a stage): 256 x 256
+// (128 KiB of LDS, one workgroup per CU, each wave 64 x 128) multiplies a
+// little faster per tile, 192 x 128 (80 KiB, two per CU) leaves less of its
+// last tiles empty, so it is taken where its rounded area is under 0.85 of the
+// other's.  Measured at Ch = 128, us, 256 x 256 / 192 x 128: Np 1024 268 / 309,
+// 960 250 / 269, 896 222 / 213, 832 202 / 199, 704 124 / 128, 640 108 / 103,
+// 576 90 / 72, 512 47 / 53, 448 39 / 47, 384 33 / 29, 320 28 / 24.  Where a
+// channel is one tile: Np 256 as 256 x 128 (13.3, against 15.4 as 256 x 256
+// with a workgroup for only half the CUs), 192 as 192 x 128 (9.7, against
+// 10.7 as 128 x 128), up to 128 as 128 x 128 (8.8; Ch = 384 10.4 against 11.7
+// as 192 x 128).  With planes rounded up to 128 and 128 x 128 tiles N = 300
+// took 44 us and N = 517 at Ch = 384 327 (now 24 and 195).
+// ODDE_CONTRACT_TILE=256x256, 256x128, 192x128 or 128x128 overrides the
+// choice (tuning).
+enum ContractTile { kTile128 = 1, kTile192x128, kTile256x128, kTile256 };
 inline int contract_tile_override() {
   static const int v = [] {
     const char* e = getenv("ODDE_CONTRACT_TILE");
     if (!e) return 0;
-    if (strcmp(e, "256x256") == 0) return 1;
-    if (strcmp(e, "256x128") == 0) return 2;
+    if (strcmp(e, "256x256") == 0) return (int)kTile256;
+    if (strcmp(e, "256x128") == 0) return (int)kTile256x128;
+    if (strcmp(e, "192x128") == 0) return (int)kTile192x128;
+    if (strcmp(e, "128x128") == 0) return (int)kTile128;
     return 0;
   }();
   return v;
 }
 
-inline void launch_contract_big(const ContractArgs<bf16>& k, int np, int ch, hipStream_t st) {
+inline int contract_tile(int np) {
+  if (np <= 128) return kTile128;
+  if (np <= 192) return kTile192x128;
+  if (np <= 256) return kTile256x128;
+  const int64_t a256 = (int64_t)round_up(np, 256) * round_up(np, 256);
+  const int64_t a192 = (int64_t)round_up(np, 192) * round_up(np, 128);
+  return a192 * 20 < a256 * 17 ? kTile192x128 : kTile256;
+}
+
+inline void launch_contract(const ContractArgs<bf16>& k, hipStream_t st) {
+  const int np = k.np, ch = k.ch;
   const int ov = contract_tile_override();
-  // 256 x 256 from Np = 768 up (N = 768: 0.152 -> 0.138 ms against 256 x 128)
-  if (ov == 1 || (ov == 0 && np >= 768)) {
-    const int tiles = (np / 256) * (np / 256);
-    hipLaunchKernelGGL((trimul_contract_big_kernel<256, 256, 4, 2, 64, true>), dim3(tiles * ch),
-                       dim3(512), 0, st, k);
+  auto grid = [&](int tx, int ty) {
+    return dim3((unsigned)(((np + tx - 1) / tx) * ((np + ty - 1) / ty) * ch));
+  };
+  switch (ov ? ov : contract_tile(np)) {
+    case kTile256:
+      hipLaunchKernelGGL((trimul_contract_big_kernel<256, 256, 4, 2, 64, true>), grid(256, 256),
+                         dim3(512), 0, st, k);
+      break;
+    case kTile256x128:
+      hipLaunchKernelGGL((trimul_contract_big_kernel<256, 128, 4, 3, 32>), grid(256, 128),
+                         dim3(512), 0, st, k);
+      break;
+    case kTile192x128:
+      hipLaunchKernelGGL((trimul_contract_big_kernel<192, 128, 4, 2, 64, true>), grid(192, 128),
+                         dim3(512), 0, st, k);
+      break;
+    default:
+      hipLaunchKernelGGL((trimul_contract_big_kernel<128, 128, 4, 2, 64, true>), grid(128, 128),
+                         dim3(512), 0, st, k);
+  }
+}
+// fp32: 64 x 64 tiles fit every Np and give four times the workgroups (Np 128:
+// 12.1 us against 17.6 with 128 x 128, 384: 143 / 147; N = 300 89 us, against
+// 163 over planes rounded up to 128); 128 x 128 reads each operand half as
+// often from L2 and is ahead from Np = 512 (297 / 315, 640: 575 / 590).
+inline void launch_contract(const ContractArgs<float>& k, hipStream_t st) {
+  const int np = k.np;
+  if (np % 128 == 0 && np >= 512) {
+    hipLaunchKernelGGL((trimul_contract_f32_kernel<128>), dim3((np / 128) * (np / 128) * k.ch),
+                       dim3(256), 0, st, k);
   } else {
-    const int tiles = (np / 256) * (np / 128);
-    hipLaunchKernelGGL((trimul_contract_big_kernel<256, 128, 4, 3, 32>), dim3(tiles * ch), dim3(512),
-                       0, st, k);
+    hipLaunchKernelGGL((trimul_contract_f32_kernel<64>), dim3((np / 64) * (np / 64) * k.ch),
+                       dim3(256), 0, st, k);
   }
 }
 
@@ -403,16 +475,8 @@ __global__ __launch_bounds__(512) void trimul_contract_x3_kernel(ContractArgs<bf
   using S = GemmShape<TX, TY, WX, 64>;
   __shared__ __attribute__((aligned(16))) bf16 sm[2 * S::STAGE_ELEMS];
   const int TXn = a.np / TX, TYn = a.np / TY;
-  const int tiles = TXn * TYn;
-  int bid = blockIdx.x, c, tile;
-  if ((a.ch & 7) == 0) {  // all tiles of a channel on one XCD
-    const int xcd = bid & 7, local = bid >> 3;
-    c = (local / tiles) * 8 + xcd;
-    tile = local % tiles;
-  } else {
-    c = bid / tiles;
-    tile = bid % tiles;
-  }
+  int c, tile;
+  contract_tile_map(blockIdx.x, a.ch, TXn * TYn, c, tile);
   const int x0 = (tile / TYn) * TX, y0 = (tile % TYn) * TY;
   const int ld = 2 * a.np;
   const size_t plane = (size_t)a.np * ld;
@@ -1079,13 +1143,14 @@ __global__ __launch_bounds__(512) void trimul_proj_wide_kernel(TrimulWideProjArg
   static_assert(WideShape::MX == 4 && kWTX / kWWX == 64, "one 64-pair line per channel and wave");
   const int64_t mw = x0 + wx * (kWTX / kWWX);
   const int x = (int)(mw / np), yw = (int)(mw % np);
+  if (x >= a.n) return;  // rows past n * np (the last row tiles)
   float mk[2][8];
 #pragma unroll
   for (int hh = 0; hh < 2; ++hh)
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       const int y = yw + 32 * hh + 8 * g + e;
-      mk[hh][e] = (x < a.n && y < a.n)
+      mk[hh][e] = y < a.n
                       ? (a.mask ? a.mask[(int64_t)x * a.m_s0 + (int64_t)y * a.m_s1] : 1.0f)
                       : 0.f;
     }
@@ -1140,8 +1205,9 @@ __global__ __launch_bounds__(512) void trimul_out_wide_kernel(TrimulWideOutArgs<
   gemm_nt_mainloop<kWTX, kWTY, kWWX, kWNS, true, kWKC>(
       [&](int r) {
         const int64_t m = x0 + r;  // the incoming form's z rows were normalised transposed
-        const int64_t zr = a.zn_transposed ? (m % np) * np + m / np : m;
-        return a.zn + zr * C;
+        if (!a.zn_transposed) return a.zn + m * C;
+        const int x = (int)(m / np), y = (int)(m % np);
+        return a.zn + (x < a.n && y < a.n ? (int64_t)y * np + x : 0) * C;
       },
       [&](int r) { return a.wg + (size_t)(y0 + r) * C; }, C, sm, accg);
   const int w = wave_id(), l = lane_id(), g = l >> 4, r16 = l & 15;
@@ -1188,6 +1254,17 @@ bool trimul_ws_shape(int c, int ch, int dt) {
   return dt == ODDE_BF16 && ((c == 128 && ch == 128) || (c == 64 && (ch == 64 || ch == 128)));
 }
 
+// The three-part contraction multiplies 256 x 256 tiles, where N rounded up
+// to 128 is a multiple of 256; other sizes contract true fp32 products.
+bool trimul_x3(int n, int dt) { return dt == ODDE_F32X3 && round_up(n, 128) % 256 == 0; }
+// Rows of the A, B and P planes: 64 pairs per projection tile.  The planes'
+// area and the contraction grow with Np^2 and Np^3 (N = 300: 320 against 384
+// is 1.4 and 1.7 times less).
+int trimul_np(int n, int dt) { return round_up(n, trimul_x3(n, dt) ? 256 : 64); }
+// Pair rows (x < n, all Np columns) of the wide path's GEMMs: row tiles of
+// 256 in multiples of 8 (one per XCD).
+int64_t trimul_wide_rows(int n, int np) { return ((int64_t)n * np + 2047) / 2048 * 2048; }
+
 struct TrimulWs {
   void* A; void* B; void* P; void* zn;
   bf16* wfold; float* wsum; float* wbias;  // LN_out folded into W_z (ws shapes)
@@ -1198,7 +1275,7 @@ struct TrimulWs {
 };
 
 TrimulWs carve_trimul(void* base, uint64_t size, int n, int c, int ch, int dt) {
-  const int np = round_up(n, 128);
+  const int np = trimul_np(n, dt);
   const uint64_t plane = (uint64_t)ch * np * np * dtype_size(dt);
   Carver cv(base, size);
   TrimulWs w;
@@ -1206,8 +1283,9 @@ TrimulWs carve_trimul(void* base, uint64_t size, int n, int c, int ch, int dt) {
   w.B = cv.take<char>(plane);
   w.P = cv.take<char>(plane);
   // the wide path's LN_in(z) rows (its LN_out(P) rows reuse A after the
-  // contraction)
-  w.zn = trimul_wide(c, ch, dt) ? cv.take<char>((uint64_t)np * np * c * 2) : nullptr;
+  // contraction; the rows past n * np that the last row tiles read, fewer
+  // than 2048 and so than np * np, lie in A and B)
+  w.zn = trimul_wide(c, ch, dt) ? cv.take<char>((uint64_t)trimul_wide_rows(n, np) * c * 2) : nullptr;
   const bool fold = trimul_ws_shape(c, ch, dt);
   w.wfold = fold ? cv.take<bf16>((uint64_t)c * ch) : nullptr;
   w.wsum = fold ? cv.take<float>(c) : nullptr;
@@ -1221,25 +1299,25 @@ TrimulWs carve_trimul(void* base, uint64_t size, int n, int c, int ch, int dt) {
 
 template <typename ZT>
 int run_trimul_wide(const odde_trimul_args* a, const TrimulWs& ws, hipStream_t st) {
-  const int n = a->n, C = a->c, ch = a->c_hidden, np = round_up(n, 128);
+  const int n = a->n, C = a->c, ch = a->c_hidden, np = trimul_np(n, ODDE_BF16);
   const bool outgoing = a->outgoing != 0;
   const int64_t vs0 = outgoing ? a->z_s0 : a->z_s1, vs1 = outgoing ? a->z_s1 : a->z_s0;
-  const int64_t rows = (int64_t)np * np;             // a multiple of 16384
+  const int64_t rows = trimul_wide_rows(n, np);
   const int row_tiles = (int)(rows / kWTX);          // a multiple of 8
   bf16* zn = static_cast<bf16*>(ws.zn);
   {
     LaunchScope ls(ODDE_K_TRIMUL_PROJ, st);
-    const int lg = (int)std::min<int64_t>(rows / 16, 4096);
+    const int lg = (int)std::min<int64_t>((int64_t)n * np / 16, 4096);
     const ZT* z = static_cast<const ZT*>(a->z);
     if (C == 128)
-      hipLaunchKernelGGL((ln_view_bf16_kernel<ZT, 128>), dim3(lg), dim3(256), 0, st, z, vs0, vs1, n,
-                         np, np, a->norm_in_weight, a->norm_in_bias, a->eps, zn);
+      hipLaunchKernelGGL((ln_view_bf16_kernel<ZT, 128>), dim3(lg), dim3(256), 0, st, z, vs0, vs1, n, n,
+                         np, a->norm_in_weight, a->norm_in_bias, a->eps, zn);
     else if (C == 256)
-      hipLaunchKernelGGL((ln_view_bf16_kernel<ZT, 256>), dim3(lg), dim3(256), 0, st, z, vs0, vs1, n,
-                         np, np, a->norm_in_weight, a->norm_in_bias, a->eps, zn);
+      hipLaunchKernelGGL((ln_view_bf16_kernel<ZT, 256>), dim3(lg), dim3(256), 0, st, z, vs0, vs1, n, n,
+                         np, a->norm_in_weight, a->norm_in_bias, a->eps, zn);
     else
-      hipLaunchKernelGGL((ln_view_bf16_kernel<ZT, 384>), dim3(lg), dim3(256), 0, st, z, vs0, vs1, n,
-                         np, np, a->norm_in_weight, a->norm_in_bias, a->eps, zn);
+      hipLaunchKernelGGL((ln_view_bf16_kernel<ZT, 384>), dim3(lg), dim3(256), 0, st, z, vs0, vs1, n, n,
+                         np, a->norm_in_weight, a->norm_in_bias, a->eps, zn);
     TrimulWideProjArgs p;
     p.zn = zn;
     p.wp = static_cast<const bf16*>(a->p_in_weight);
@@ -1260,19 +1338,14 @@ int run_trimul_wide(const odde_trimul_args* a, const TrimulWs& ws, hipStream_t s
   k.np = np; k.ch = ch;
   {
     LaunchScope ls(ODDE_K_TRIMUL_CONTRACT, st);
-    if (np % 256 == 0) {
-      launch_contract_big(k, np, ch, st);
-    } else {
-      const int tiles = (np / 128) * (np / 128);
-      hipLaunchKernelGGL((trimul_contract_kernel<bf16>), dim3(tiles * ch), dim3(256), 0, st, k);
-    }
+    launch_contract(k, st);
     int rc = check_launch("trimul_contract");
     if (rc) return rc;
   }
   {
     LaunchScope ls(ODDE_K_TRIMUL_OUT, st);
     bf16* pn = static_cast<bf16*>(ws.A);  // A is dead after the contraction
-    const dim3 tg(np / 64, np);
+    const dim3 tg(np / 64, n);
     switch (ch) {
       case 64: hipLaunchKernelGGL((ln_transpose_bf16_kernel<64>), tg, dim3(256), 0, st, k.P, np, n,
                                   a->norm_out_weight, a->norm_out_bias, a->eps, pn); break;
@@ -1342,25 +1415,27 @@ template <typename ZT, typename CT, int kC, bool kX3Out = false, bool kX3Mul = f
 void launch_tp(const TrimulProjArgs<ZT, CT>& p, hipStream_t st) {
   // fp32 weights are read from L2 per fragment: more row blocks per wave as
   // registers allow (4 up to C = 128, 2 at C = 256), once the grid stays
-  // large enough (np >= 256: np^2 / 256 workgroups and more)
+  // large enough (N > 128); rows past N of the last block are rows of the
+  // planes (Np is a multiple of kRB)
   constexpr int kRB = sizeof(CT) != 4 ? 1 : kC <= 4 ? 4 : kC <= 8 ? 2 : 1;
   if constexpr (sizeof(CT) == 4 && kC <= 4) {
-    // f32 data from Np = 256: the weights staged in LDS (kSRB row blocks
+    // f32 data from N = 129: the weights staged in LDS (kSRB row blocks
     // per wave)
-    if (p.np >= 256 && !trimul_proj_f32_plain()) {
-      dim3 grid(p.np / 64, p.np / kSRB);
+    if (p.n > 128 && !trimul_proj_f32_plain()) {
+      dim3 grid(p.np / 64, (p.n + kSRB - 1) / kSRB);
       hipLaunchKernelGGL((trimul_proj_kernel<ZT, CT, kC, kSRB, kX3Out, kX3Mul, true>), grid,
                          dim3(256), 0, st, p);
       return;
     }
   }
-  if (kX3Out || (kRB > 1 && p.np >= 256)) {
-    dim3 grid(p.np / 64, p.np / kRB, proj_split((int64_t)(p.np / 64) * (p.np / kRB), p.ch / 16));
+  if (kX3Out || (kRB > 1 && p.n > 128)) {
+    const int rows = (p.n + kRB - 1) / kRB;
+    dim3 grid(p.np / 64, rows, proj_split((int64_t)(p.np / 64) * rows, p.ch / 16));
     hipLaunchKernelGGL((trimul_proj_kernel<ZT, CT, kC, kRB, kX3Out, kX3Mul>), grid, dim3(256), 0,
                        st, p);
     return;
   }
-  dim3 grid(p.np / 64, p.np, proj_split((int64_t)(p.np / 64) * p.np, p.ch / 16));
+  dim3 grid(p.np / 64, p.n, proj_split((int64_t)(p.np / 64) * p.n, p.ch / 16));
   hipLaunchKernelGGL((trimul_proj_kernel<ZT, CT, kC, 1, false, kX3Mul>), grid, dim3(256), 0, st, p);
 }
 template <typename ZT, int kC>
@@ -1374,7 +1449,7 @@ void launch_tp_f32(const TrimulProjArgs<ZT, float>& p, bool x3out, bool x3mul, h
 // registers (bf16, C and Ch in {64, 128}); false otherwise.
 template <typename ZT, typename CT, int kC, int kCH>
 void launch_tp_ws_t(const TrimulProjArgs<ZT, CT>& p, hipStream_t st) {
-  const int ntiles = p.np * (p.np / kTileRows);
+  const int ntiles = p.n * (p.np / kTileRows);
   static const int resident =
       resident_grid(reinterpret_cast<const void*>(&trimul_proj_ws_kernel<ZT, CT, kC, kCH>), 256);
   hipLaunchKernelGGL((trimul_proj_ws_kernel<ZT, CT, kC, kCH>), dim3(min(ntiles, resident)),
@@ -1482,7 +1557,7 @@ bool dispatch_to(const TrimulOutArgs<ZT, CT>& p, int ch, bool x3, hipStream_t st
 template <typename ZT, typename CT>
 int run_trimul(const odde_trimul_args* a, hipStream_t st) {
   const int n = a->n, C = a->c, ch = a->c_hidden;
-  const int np = round_up(n, 128);
+  const int np = trimul_np(n, a->compute_dtype);
   TrimulWs ws = carve_trimul(a->workspace, a->workspace_bytes, n, C, ch, a->compute_dtype);
   if constexpr (sizeof(CT) == 2) {
     if (trimul_wide(C, ch, a->compute_dtype)) return run_trimul_wide<ZT>(a, ws, st);
@@ -1503,10 +1578,9 @@ int run_trimul(const odde_trimul_args* a, hipStream_t st) {
   p.A = static_cast<CT*>(ws.A); p.B = static_cast<CT*>(ws.B);
   p.n = n; p.np = np; p.ch = ch; p.eps = a->eps;
   // the three-part fp32 form: the projections' and the output's products
-  // always, the contraction where its tiles fit (Np a multiple of 256;
-  // otherwise true fp32 products)
+  // always, the contraction where trimul_x3 says so
   const bool x3mul = sizeof(CT) == 4 && a->compute_dtype == ODDE_F32X3;
-  const bool x3 = x3mul && np % 256 == 0;
+  const bool x3 = trimul_x3(n, a->compute_dtype);
   const CT* w_z = static_cast<const CT*>(a->p_out_weight);
   const CT* w_go = static_cast<const CT*>(a->g_out_weight);
   if (x3mul) {
@@ -1556,16 +1630,8 @@ int run_trimul(const odde_trimul_args* a, hipStream_t st) {
       const int tiles = (np / 256) * (np / 256);
       hipLaunchKernelGGL(trimul_contract_x3_kernel, dim3(tiles * ch), dim3(512), 0, st, kb,
                          static_cast<float*>(ws.P));
-    } else if constexpr (sizeof(CT) == 2) {
-      if (np % 256 == 0) {
-        launch_contract_big(k, np, ch, st);
-      } else {
-        const int tiles = (np / 128) * (np / 128);
-        hipLaunchKernelGGL((trimul_contract_kernel<CT>), dim3(tiles * ch), dim3(256), 0, st, k);
-      }
     } else {
-      const int tiles = (np / 128) * (np / 128);
-      hipLaunchKernelGGL((trimul_contract_kernel<CT>), dim3(tiles * ch), dim3(256), 0, st, k);
+      launch_contract(k, st);
     }
     int rc = check_launch("trimul_contract");
     if (rc) return rc;

@@ -73,3 +73,31 @@ def test_block_sizes(n):
                          triangle_attention="hip", inplace_safe=True)
     assert_bf16(zb - z.to(DEV), ze - z, f"block bf16 n={n} z update")
     assert_bf16(sb - s.to(DEV), se - s, f"block bf16 n={n} s update")
+
+
+@pytest.mark.parametrize("n,c", [(66, 64), (129, 64), (191, 64), (256, 64), (319, 64), (384, 64),
+                                 (385, 64), (450, 64), (513, 64), (577, 64), (190, 384),
+                                 (321, 384), (449, 384)])
+@pytest.mark.parametrize("outgoing", [True, False])
+def test_multiplication_plane_sizes(n, c, outgoing):
+    """Planes rounded up to 64 and every tile of the contraction, with whole
+    and partial last tiles (Np 128 to 640), over a workspace of NaN: rows that
+    no projection writes must not reach the result."""
+    say(f"[gpu] plane sizes n={n} c={c} out={outgoing}")
+    z = torch.randn(n, n, c, generator=torch.Generator().manual_seed(n + c))
+    mask = token_pair_mask(n, 2)
+    cls = TriangleMultiplicationOutgoing if outgoing else TriangleMultiplicationIncoming
+    mod = seeded(cls(c, c), n, 0.1 if c == 64 else 0.05)
+    exp = ref.triangle_multiplication(z, mask, params_of(mod), outgoing=outgoing)
+    mod, zd, md = mod.to(DEV), z.to(DEV), mask.to(DEV)
+
+    def run(autocast):
+        torch.cuda.empty_cache()
+        dirty = torch.full((1 << 28,), float("nan"), device=DEV)
+        del dirty  # its block serves the call's workspace
+        with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16, enabled=autocast):
+            return mod(zd, md, triangle_multiplicative="hip")
+
+    assert_bf16(run(True), exp, f"planes bf16 n={n} c={c} out={outgoing}")
+    if c == 64:
+        assert_fp32(run(False), exp, f"planes n={n} c={c} out={outgoing}")
