@@ -50,9 +50,9 @@
 
 #include <type_traits>
 
+#include "astat.hpp"
 #include "common.hpp"
 #include "gemm.hpp"
-#include "lnpass.hpp"
 #include "rowtile.hpp"
 #include "runtime.hpp"
 
@@ -1726,10 +1726,10 @@ __global__ __launch_bounds__(256) void triatt_mflag_kernel(const float* mb, int*
 }
 
 // ---------------------------------------------------------------------------
-// 5. wide channels (bf16; C or H*32 of 256 and more): a LayerNorm pass into
-//    bf16 rows (lnpass.hpp), then NT GEMMs on the shared mainloop
-//    (gemm.hpp).  Rows are the pairs m = i * Jp + j, padded to a multiple of
-//    2048 (rows past n * Jp are never stored).
+// 5. wide channels (bf16; C or H*32 of 256 and more): the LayerNorm and all
+//    projections in one row-stationary GEMM (astat.hpp), the output as an NT
+//    GEMM (gemm.hpp).  Rows are the pairs m = i * Jp + j, padded to a multiple
+//    of 2048 (rows past n * Jp are never stored).
 // ---------------------------------------------------------------------------
 constexpr int kWTX = 256, kWTY = 128, kWWX = 4, kWNS = 3, kWKC = 32;
 using WideShape = GemmShape<kWTX, kWTY, kWWX, kWKC>;
@@ -1740,182 +1740,186 @@ __device__ __forceinline__ void wide_tile_map(int L, int ncol, int& rt, int& ct)
   ct = s % ncol;
 }
 
-// Mask outputs (mb, mflag, keep) and the triangle bias of 64 pairs (i, j0..)
-// from the normalised rows, as in the register projection kernel: a
-// workgroup of 4 waves, 16 pairs per wave.
-template <typename ZT, int kC>
-__global__ __launch_bounds__(256) void triatt_bias_mask_wide_kernel(TriattProjArgs<ZT, bf16> a,
-                                                                    const bf16* zn) {
-  constexpr int C = kC * 32;
-  const int i = blockIdx.y;
-  const int w = wave_id(), l = lane_id(), g = l >> 4, r16 = l & 15;
+// Mask outputs (mb, mflag, keep) and the triangle bias of the wave's 16 MB pairs
+// (row, jw ..) from its normalised rows.  mv: lane l's additive mask value,
+// kp: 1 if its key is kept (lanes < 16 MB).
+template <int MB, int KT, typename ZT>
+__device__ __forceinline__ void triatt_bias_mask_rows(const TriattProjArgs<ZT, bf16>& a,
+                                                      const Frag<bf16> (&A)[MB][KT], int row,
+                                                      int jw, int l, float mv, float kp) {
+  constexpr int C = KT * 32;
+  const int g = l >> 4, r16 = l & 15;
   const int H = a.heads, jp = a.jp;
-  const int j0 = blockIdx.x * 64 + w * 16;
-  const int jl = j0 + r16;
-  const bool valid = jl < a.n;
-  Frag<bf16> x[kC];
-  const bf16* row = zn + ((size_t)i * jp + jl) * C + 8 * g;
+  const size_t blk = (size_t)row * (jp >> 5) + (jw >> 5);  // first 32-key block
+  const unsigned long long masked = __ballot(mv != 0.f);
+  const int s = l & 31;
+  const float ks = __shfl(kp, (l & 32) + slot_key(s >> 3, s & 7), 64);
+  if (l < 16 * MB) {
+    a.mb[(size_t)row * jp + jw + l] = mv;
+    a.keep[blk * 32 + l] = (bf16)ks;
+  }
+  if (l < MB / 2) a.mflag[blk + l] = (unsigned)(masked >> (32 * l)) != 0u;
+  // channel h = r16 (< H), pairs 16 i + 4 g .. + 3 -> bias[h][row][..]
+  const bf16* wb = a.wb + (size_t)min(r16, H - 1) * C + 8 * g;
+  f32x4 ab[MB];
 #pragma unroll
-  for (int t = 0; t < kC; ++t) x[t].load(row + 32 * t);
-
-  __shared__ float keep_s[64];
-  __shared__ int wmasked[4];
-  float mv = -INFINITY, kp = 0.f;
-  if (valid) {
-    const float m = a.mask ? a.mask[(int64_t)i * a.m_s0 + (int64_t)jl * a.m_s1] : 1.0f;
-    mv = (m - 1.0f) * a.mask_inf;
-    kp = m == 1.0f ? 1.f : 0.f;
-  }
-  if (g == 0) {
-    a.mb[(size_t)i * jp + jl] = mv;
-    keep_s[w * 16 + r16] = kp;
-  }
-  const bool any_masked = __any(mv != 0.f);
-  if (l == 0) wmasked[w] = any_masked ? 1 : 0;
-  __syncthreads();
-  if (threadIdx.x < 2) {
-    const int b = threadIdx.x;  // 32-key block b of this 64-key tile = waves 2b, 2b+1
-    a.mflag[(size_t)i * (jp >> 5) + blockIdx.x * 2 + b] = wmasked[2 * b] | wmasked[2 * b + 1];
-  }
-  if (threadIdx.x < 64) {
-    const int t = threadIdx.x, kb = t >> 5, s = t & 31;
-    a.keep[((size_t)i * (jp >> 5) + blockIdx.x * 2 + kb) * 32 + s] =
-        (bf16)keep_s[kb * 32 + slot_key(s >> 3, s & 7)];
-  }
-  // triangle bias: channel h = r16 (< H), rows j0+4g .. +3 -> bias[h][i][..]
-  f32x4 ab = {0.f, 0.f, 0.f, 0.f};
+  for (int i = 0; i < MB; ++i) ab[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int t = 0; t < kC; ++t) {
+  for (int t = 0; t < KT; ++t) {
     Frag<bf16> f;
-    load_w_frag(a.wb, C, 0, H, t, f);
-    mma(ab, x[t], f);
+    f.load(wb + 32 * t);
+#pragma unroll
+    for (int i = 0; i < MB; ++i) mma(ab[i], A[i][t], f);
   }
-  const float sc = kLog2e;
-  const int jb = j0 + 4 * g;
-  const float bm = group_max_fast(fmaxf(fmaxf(ab[0], ab[1]), fmaxf(ab[2], ab[3])) * sc);
-  if (r16 < H) {
-    store4(a.bias + ((size_t)r16 * jp + i) * jp + jb, ab[0] * sc, ab[1] * sc, ab[2] * sc,
-           ab[3] * sc);
-    if (g == 0) atomicMax(&a.bmax[r16 * jp + i], fkey(bm));
+  float bm = -INFINITY;
+  float* dst = a.bias + ((size_t)r16 * jp + row) * jp + jw + 4 * g;
+#pragma unroll
+  for (int i = 0; i < MB; ++i) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      ab[i][e] *= kLog2e;
+      bm = fmaxf(bm, ab[i][e]);
+    }
+    if (r16 < H) store4(dst + 16 * i, ab[i][0], ab[i][1], ab[i][2], ab[i][3]);
   }
+  bm = group_max_fast(bm);
+  if (r16 < H && g == 0) atomicMax(&a.bmax[r16 * jp + row], fkey(bm));
 }
 
-// q, k, v, gate as one NT GEMM of the normalised rows with the weight rows
-// [W_q | W_k | W_v | W_g] (H*32 each, a multiple of the 128-row column tile,
-// so a tile is one of the four).  q, k, gate: one pair and four consecutive
-// channels per lane (8-byte stores into [I][H][Jp][32]); v: one channel and
-// four consecutive pairs per lane (8-byte stores into the fragment-ordered
-// V layout), zeroed on masked keys of rows that keep a key.  k also yields
-// the per-(row, head) maximum key norm for the fast core's bound.
-template <typename ZT>
-__global__ __launch_bounds__(512) void triatt_qkvg_wide_kernel(TriattProjArgs<ZT, bf16> a,
-                                                               const bf16* zn, int C, int ncol) {
-  __shared__ __attribute__((aligned(16))) bf16 sm[kWNS * WideShape::STAGE_ELEMS];
+// q, k, v, gate as one row-stationary GEMM (astat.hpp) of the normalised rows
+// with the weight rows [W_q | W_k | W_v | W_g]: a stage is one head of one of
+// the four (kType 0 .. 3).  LDS row 16 j + m holds channel 8 (m >> 2) + 4 j +
+// (m & 3) of the head.  q, k, gate: a lane's results of the two row blocks are
+// 8 consecutive channels of one pair (16-byte stores into [I][H][Jp][32], a
+// wave's store instruction 1 KiB on end); v: one channel, and the keys of row
+// blocks i and i + 1 that form a 16-byte slot group of the fragment-ordered V
+// layout, zeroed on masked keys of rows that keep a key.  k also yields the
+// per-(row, head) maximum key norm for the fast core's bound.  This is heads
+// h0 .. h0 + nst - 1 of one of the four, for the wave's 64 pairs (row, jw ..);
+// vk: the value factors of those pairs (LDS).
+template <int kType, int MB, int KT, typename ZT>
+__device__ __forceinline__ void qkvg_wide_type(const TriattProjArgs<ZT, bf16>& a,
+                                               const Frag<bf16> (&A)[MB][KT], int row, int jw,
+                                               int h0, int nst, bf16* sm,
+                                               const float* vk_s) {
+  constexpr int C = KT * 32;
+  const int H = a.heads, jp = a.jp;
+  const int w = __builtin_amdgcn_readfirstlane(wave_id());
+  const int l = astat_lane(), g = l >> 4, r16 = l & 15;
+  const bool live = row < a.n;
+  const bf16* W = (kType == 0 ? a.wq : kType == 1 ? a.wk : kType == 2 ? a.wv : a.wg) +
+                  (size_t)(h0 * 32 + 16 * (w & 1) + 4 * (w >> 1)) * C;
+  bf16* plane = kType == 0 ? a.q : kType == 1 ? a.k : kType == 2 ? a.v : a.gate;
+  // head h0 of the wave's 64 pairs: 64 x 32 elements on end in either layout
+  bf16* dst = plane + (((size_t)row * H + h0) * jp + jw) * 32;
+  const int lo = kType == 2 ? (int)(vperm_offset(0, 0, H, jp, 4 * g, 8 * (r16 >> 2) + (r16 & 3)))
+                            : r16 * 32 + 8 * g;
+  unsigned* kmax = a.kmax + (size_t)row * H + h0;
+  astat_loop<KT, MB>(
+      nst, live, sm, l, [&](int st) { return W + (size_t)st * 32 * C; },
+      [](int r) { return 8 * (r >> 2) + (r & 3); },
+      [&](int st, const bf16* buf) __attribute__((always_inline)) {
+        f32x4 acc[MB][2];
+        astat_mult<MB, KT, kType != 2>(buf, l, A, acc);
+        bf16* d = dst + (size_t)st * jp * 32;
+        if constexpr (kType == 2) {
+          // keys jw + 16 i + 4 g .. + 3 and the same + 16: one slot group of
+          // key block i / 2, channel half j
+#pragma unroll
+          for (int i = 0; i < MB; i += 2) {
+            float vk[8];
+            load4(vk_s + 16 * i + 4 * g, vk);
+            load4(vk_s + 16 * i + 16 + 4 * g, vk + 4);
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+              bf16x8 v8;
+#pragma unroll
+              for (int e = 0; e < 4; ++e) {
+                v8[e] = (bf16)(acc[i][j][e] * vk[e]);
+                v8[4 + e] = (bf16)(acc[i + 1][j][e] * vk[4 + e]);
+              }
+              *reinterpret_cast<bf16x8*>(d + lo + (i + j) * 512) = v8;
+            }
+          }
+        } else {
+          float knm = 0.f;
+#pragma unroll
+          for (int i = 0; i < MB; ++i) {
+            bf16x8 v8;
+            float ss = 0.f;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+              const float v = acc[i][e >> 2][e & 3];
+              if constexpr (kType == 0) v8[e] = (bf16)(v * a.q_scale);
+              if constexpr (kType == 1) {
+                v8[e] = (bf16)v;
+                ss += v * v;
+              }
+              if constexpr (kType == 3) v8[e] = (bf16)sigmoidf_(v);
+            }
+            store_stream(reinterpret_cast<bf16x8*>(d + lo + i * 512), v8);
+            if constexpr (kType == 1) knm = fmaxf(knm, sqrtf(group_sum_fast(ss)));
+          }
+          if constexpr (kType == 1) {
+            const float v = lanes16_max(knm);
+            if (l == 0) atomicMax(kmax + st, __float_as_uint(v));
+          }
+        }
+      });
+}
+
+// gridDim: row tiles x csplit (a divisor of 4 H), each workgroup 4 H / csplit of
+// the stages [q heads | k heads | v heads | gate heads].  The LayerNorm is
+// fused into the row loads and the first split adds the bias and mask outputs,
+// which were two more passes over the rows: C = 384, N = 640, all three
+// 1006 -> 635 us (1.9 GB moved, 760 TF/s over the whole).
+template <int MB, int KT, typename ZT>
+__global__ __launch_bounds__(256, 2) void triatt_qkvg_wide_kernel(TriattProjArgs<ZT, bf16> a,
+                                                                  int csplit) {
+  constexpr int C = KT * 32;
+  __shared__ __attribute__((aligned(16))) bf16 sm[AstatShape<MB, KT>::LDS];
   int rt, ct;
-  wide_tile_map(blockIdx.x, ncol, rt, ct);
-  const int H = a.heads, HD = H * 32, jp = a.jp, n = a.n;
-  const int64_t x0 = (int64_t)rt * kWTX;
-  const int per = HD / kWTY, type = ct / per, o0 = (ct % per) * kWTY;
-  const bf16* W = type == 0 ? a.wq : type == 1 ? a.wk : type == 2 ? a.wv : a.wg;
-  const int w = wave_id(), l = lane_id(), g = l >> 4, r16 = l & 15;
-  const int wx = w % kWWX, wy = w / kWWX;
-  auto arow = [&](int r) { return zn + (x0 + r) * C; };
-  auto brow = [&](int r) { return W + (size_t)(o0 + r) * C; };
-  // q, k, gate: within each 32 weight rows (one head), row block 2p + b, MFMA
-  // row m is channel 8 (m >> 2) + 4 b + (m & 3), so a lane's results of the
-  // head's two row blocks are 8 consecutive channels (one 16-byte store)
-  auto brow_perm = [&](int r) {
-    const int m = r & 15;
-    return W + (size_t)(o0 + (r & ~31) + 8 * (m >> 2) + 4 * ((r >> 4) & 1) + (m & 3)) * C;
+  wide_tile_map(blockIdx.x, csplit, rt, ct);
+  const int H = a.heads, jp = a.jp, n = a.n;
+  const int64_t x0 = (int64_t)rt * (64 * MB);
+  if (x0 >= (int64_t)n * jp) return;
+  const int w = __builtin_amdgcn_readfirstlane(wave_id()), r16 = lane_id() & 15;
+  // the wave's pairs lie in one row (Jp is a multiple of 64)
+  const int64_t mw = x0 + 16 * MB * w;
+  const int row = (int)(mw / jp), jw = (int)(mw % jp);
+  const bool live = row < n;
+  float* vk_s = astat_row_floats<KT>(sm) + 16 * MB * w;
+  Frag<bf16> A[MB][KT];
+  const ZT* zr = a.z + (int64_t)(live ? row : 0) * a.z_s0;
+#pragma unroll
+  for (int i = 0; i < MB; ++i) {
+    const int j = jw + 16 * i + r16;
+    const bool valid = live && j < n;
+    astat_ln_rows<MB == 4, KT>(zr + (int64_t)(valid ? j : 0) * a.z_s1, valid, a.ln_w, a.ln_b, a.eps, A[i]);
+  }
+  const int l = astat_lane();
+  if (live) {
+    const int key = jw + l;
+    float mv = -INFINITY, kp = 0.f;
+    if (l < 16 * MB && key < n) {
+      const float m = a.mask ? a.mask[(int64_t)row * a.m_s0 + (int64_t)key * a.m_s1] : 1.0f;
+      mv = (m - 1.0f) * a.mask_inf;
+      kp = m == 1.0f ? 1.f : 0.f;
+    }
+    if (l < 16 * MB) vk_s[l] = a.anykeep[row] != 0 ? kp : 1.f;
+    if (ct == 0) triatt_bias_mask_rows<MB, KT>(a, A, row, jw, l, mv, kp);
+  }
+  astat_rows_ready<MB, KT>(A);
+  const int u0 = 4 * H / csplit * ct, u1 = u0 + 4 * H / csplit;  // stages of [q | k | v | gate]
+  auto part = [&](int type, int& h0) {  // its heads in this workgroup's stages
+    h0 = max(u0 - type * H, 0);
+    return min(u1 - type * H, H) - h0;
   };
-  f32x4 acc[WideShape::MX][WideShape::MY];
-  static_assert(WideShape::MX % 2 == 0 && WideShape::MY % 2 == 0, "row blocks pair up");
-  if (type == 2) {  // v: channel-per-lane orientation
-    gemm_nt_mainloop<kWTX, kWTY, kWWX, kWNS, false, kWKC>(arow, brow, C, sm, acc);
-    // row blocks i and i + 1 hold keys 4g..4g+3 and the same keys + 16 of a
-    // 32-key block: one 16-byte slot group of the V layout
-#pragma unroll
-    for (int i = 0; i < WideShape::MX; i += 2) {
-      const int64_t m = x0 + wx * (kWTX / kWWX) + 16 * i + 4 * g;  // pairs m .. m+3, m+16 ..
-      const int row = (int)(m / jp), jj = (int)(m % jp);
-      if (row >= n) continue;
-      float vk[8] = {1.f, 1.f, 1.f, 1.f, 1.f, 1.f, 1.f, 1.f};
-      if (a.anykeep[row] != 0) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const int key = jj + (e & 3) + 16 * (e >> 2);
-          const float mv = key < n ? (a.mask ? a.mask[(int64_t)row * a.m_s0 +
-                                                      (int64_t)key * a.m_s1]
-                                             : 1.0f)
-                                   : 0.f;
-          vk[e] = mv == 1.0f ? 1.f : 0.f;
-        }
-      }
-#pragma unroll
-      for (int j = 0; j < WideShape::MY; ++j) {
-        const int o = o0 + wy * (kWTY / WideShape::WY) + 16 * j + r16;
-        bf16x8 v8;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          v8[e] = (bf16)(acc[i][j][e] * vk[e]);
-          v8[4 + e] = (bf16)(acc[i + 1][j][e] * vk[4 + e]);
-        }
-        *reinterpret_cast<bf16x8*>(a.v + vperm_offset(row, o >> 5, H, jp, jj, o & 31)) = v8;
-      }
-    }
-    return;
-  }
-  gemm_nt_mainloop<kWTX, kWTY, kWWX, kWNS, true, kWKC>(arow, brow_perm, C, sm, acc);
-  // the wave's 64 pairs lie in one row (Jp and the offsets are multiples of 64)
-  const int64_t mw = x0 + wx * (kWTX / kWWX);
-  const int row = (int)(mw / jp);
-  if (row >= n) return;
-  const int ob = o0 + wy * (kWTY / WideShape::WY);  // the wave's 64 channels = heads ob/32, +1
-  float knm[2] = {0.f, 0.f};
-#pragma unroll
-  for (int i = 0; i < WideShape::MX; ++i) {
-    const int jj = (int)((mw + 16 * i + r16) % jp);
-    float ss[2] = {0.f, 0.f};
-#pragma unroll
-    for (int j = 0; j < WideShape::MY; j += 2) {
-      const int o = ob + 16 * j + 8 * g;  // 8 channels: block j gives o..o+3, j + 1 o+4..o+7
-      const size_t off = (((size_t)row * H + (o >> 5)) * jp + jj) * 32 + (o & 31);
-      float v[8];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        v[e] = acc[i][j][e];
-        v[4 + e] = acc[i][j + 1][e];
-      }
-      bf16x8 v8;
-      if (type == 0) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) v8[e] = (bf16)(v[e] * a.q_scale);
-        store_stream(reinterpret_cast<bf16x8*>(a.q + off), v8);
-      } else if (type == 1) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          v8[e] = (bf16)v[e];
-          ss[j >> 1] += v[e] * v[e];
-        }
-        store_stream(reinterpret_cast<bf16x8*>(a.k + off), v8);
-      } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) v8[e] = (bf16)sigmoidf_(v[e]);
-        store_stream(reinterpret_cast<bf16x8*>(a.gate + off), v8);
-      }
-    }
-    if (type == 1) {
-#pragma unroll
-      for (int hh = 0; hh < 2; ++hh) knm[hh] = fmaxf(knm[hh], sqrtf(group_sum_fast(ss[hh])));
-    }
-  }
-  if (type == 1) {
-#pragma unroll
-    for (int hh = 0; hh < 2; ++hh) {
-      const float v = lanes16_max(knm[hh]);
-      if (l == 0) atomicMax(&a.kmax[row * H + (ob >> 5) + hh], __float_as_uint(v));
-    }
-  }
+  int h0, nst;
+  if ((nst = part(0, h0)) > 0) qkvg_wide_type<0, MB, KT>(a, A, row, jw, h0, nst, sm, vk_s);
+  if ((nst = part(1, h0)) > 0) qkvg_wide_type<1, MB, KT>(a, A, row, jw, h0, nst, sm, vk_s);
+  if ((nst = part(2, h0)) > 0) qkvg_wide_type<2, MB, KT>(a, A, row, jw, h0, nst, sm, vk_s);
+  if ((nst = part(3, h0)) > 0) qkvg_wide_type<3, MB, KT>(a, A, row, jw, h0, nst, sm, vk_s);
 }
 
 // out[i][j][c] = (add ? res : 0) + o W_o^T: NT GEMM of the gated attention
@@ -2009,7 +2013,7 @@ int64_t triatt_wide_rows(int n) { return (int64_t)round_up(n * round_up(n, 64), 
 
 // wsplit (ODDE_F32X3): W_q, W_k, W_v, W_g ([HD][C] each), W_b ([H][C]) and
 // W_o ([C][HD]) split once per call into bf16 hi | lo rows
-struct TriattWs { CoreBufs c; void* gate; void* o; void* zn; char* wsplit; uint64_t bytes; };
+struct TriattWs { CoreBufs c; void* gate; void* o; char* wsplit; uint64_t bytes; };
 
 TriattWs carve_triatt(void* base, uint64_t size, int n, int heads, int cz, int dt) {
   const int jp = round_up(n, 64);
@@ -2021,7 +2025,6 @@ TriattWs carve_triatt(void* base, uint64_t size, int n, int heads, int cz, int d
   w.gate = triatt_ws(cz, heads, dt) ? nullptr : c.take<char>(per);
   // the wide path reads o as GEMM rows, whole 256-row tiles
   w.o = c.take<char>(wide ? (uint64_t)triatt_wide_rows(n) * heads * 32 * 2 : per);
-  w.zn = wide ? c.take<char>((uint64_t)triatt_wide_rows(n) * cz * 2) : nullptr;
   const uint64_t hd = (uint64_t)heads * 32;
   w.wsplit = dt == ODDE_F32X3 ? c.take<char>((5 * hd + heads) * cz * 4) : nullptr;
   w.bytes = (c.used + 255) & ~uint64_t(255);
@@ -2282,37 +2285,35 @@ void fill_core_args(TriattCoreArgs<CT>& c, const CoreBufs& b) {
 
 // Wide-channel projection: LayerNorm pass into bf16 rows, mask outputs and
 // triangle bias, then q, k, v, gate as one NT GEMM.
-template <typename ZT>
-int run_triatt_proj_wide(const TriattProjArgs<ZT, bf16>& p, const odde_triatt_args* a, bf16* zn,
-                         hipStream_t st) {
-  const int n = p.n, jp = p.jp, C = a->c, HD = p.heads * 32;
-  const int64_t rows = (int64_t)n * jp;
-  const int lg = (int)std::min<int64_t>((rows + 15) / 16, 4096);
+template <typename ZT, int MB>
+int launch_qkvg_wide(const TriattProjArgs<ZT, bf16>& p, int C, hipStream_t st) {
+  const int row_tiles = (int)(triatt_wide_rows(p.n) / (64 * MB));
+  const int csplit = astat_csplit(row_tiles, 4 * p.heads, 256);
+  const dim3 pg(row_tiles * csplit);
   switch (C) {
     case 128:
-      hipLaunchKernelGGL((ln_view_bf16_kernel<ZT, 128>), dim3(lg), dim3(256), 0, st, p.z, p.z_s0,
-                         p.z_s1, n, n, jp, p.ln_w, p.ln_b, p.eps, zn);
-      hipLaunchKernelGGL((triatt_bias_mask_wide_kernel<ZT, 4>), dim3(jp / 64, n), dim3(256), 0,
-                         st, p, zn);
+      hipLaunchKernelGGL((triatt_qkvg_wide_kernel<MB, 4, ZT>), pg, dim3(256), 0, st, p, csplit);
       break;
     case 256:
-      hipLaunchKernelGGL((ln_view_bf16_kernel<ZT, 256>), dim3(lg), dim3(256), 0, st, p.z, p.z_s0,
-                         p.z_s1, n, n, jp, p.ln_w, p.ln_b, p.eps, zn);
-      hipLaunchKernelGGL((triatt_bias_mask_wide_kernel<ZT, 8>), dim3(jp / 64, n), dim3(256), 0,
-                         st, p, zn);
+      hipLaunchKernelGGL((triatt_qkvg_wide_kernel<MB, 8, ZT>), pg, dim3(256), 0, st, p, csplit);
       break;
     case 384:
-      hipLaunchKernelGGL((ln_view_bf16_kernel<ZT, 384>), dim3(lg), dim3(256), 0, st, p.z, p.z_s0,
-                         p.z_s1, n, n, jp, p.ln_w, p.ln_b, p.eps, zn);
-      hipLaunchKernelGGL((triatt_bias_mask_wide_kernel<ZT, 12>), dim3(jp / 64, n), dim3(256), 0,
-                         st, p, zn);
+      hipLaunchKernelGGL((triatt_qkvg_wide_kernel<MB, 12, ZT>), pg, dim3(256), 0, st, p, csplit);
       break;
     default: return set_error(ODDE_EUNSUPPORTED, "triatt: c must be 128, 256 or 384 here");
   }
-  const int row_tiles = (int)(triatt_wide_rows(n) / kWTX), ncol = 4 * HD / kWTY;
-  hipLaunchKernelGGL((triatt_qkvg_wide_kernel<ZT>), dim3(row_tiles * ncol), dim3(512), 0, st, p,
-                     zn, C, ncol);
   return ODDE_OK;
+}
+template <typename ZT>
+int run_triatt_proj_wide(const TriattProjArgs<ZT, bf16>& p, int C, hipStream_t st) {
+  // 32 rows a wave while the grid is short of workgroups: half the LayerNorm
+  // in a row per wave, twice the weight reads per MFMA.  C = 384, us, 32 / 64
+  // rows (each at its best split): N = 40 27 / 41, 128 48 / 61, 200 94 / 110,
+  // 256 122 / 130, 300 181 / 179.  The split, 32 rows, at 1 / 2 / 4 / 8: N = 40
+  // (32 row tiles) 57 / 40 / 30 / 27, 128 (128) 65 / 48 / 51 / 69, 200 (400)
+  // 97 / 116 / 140 / 191.
+  if (p.n <= 256) return launch_qkvg_wide<ZT, 2>(p, C, st);
+  return launch_qkvg_wide<ZT, 4>(p, C, st);
 }
 
 template <typename ZT, typename CT>
@@ -2368,7 +2369,7 @@ int run_triatt(const odde_triatt_args* a, hipStream_t st) {
     hipLaunchKernelGGL(triatt_prep_kernel, dim3(n), dim3(256), 0, st, pa);
     if constexpr (sizeof(CT) == 2) {
       if (wide) {
-        int rc = run_triatt_proj_wide<ZT>(p, a, static_cast<bf16*>(ws.zn), st);
+        int rc = run_triatt_proj_wide<ZT>(p, C, st);
         if (rc) return rc;
       }
     }

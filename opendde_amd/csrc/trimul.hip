@@ -22,6 +22,7 @@
 //   and columns of P past N hold no value (they are read, never used)
 #include <string.h>
 
+#include "astat.hpp"
 #include "common.hpp"
 #include "gemm.hpp"
 #include "lnpass.hpp"
@@ -1093,85 +1094,82 @@ __device__ __forceinline__ void wide_tile_map(int L, int ncol, int& rt, int& ct)
 }
 
 struct TrimulWideProjArgs {
-  const bf16* zn;   // [Np^2][C] LN_in rows in the projection's view order
+  const bf16* zn;   // [n * Np][C] LN_in rows in the projection's view order
   const bf16* wp;   // [2*Ch][C] (a_p rows, then b_p rows)
   const bf16* wg;   // [2*Ch][C]
   const float* mask;
   int64_t m_s0, m_s1;
   bf16* A;          // [Ch][Np][Np]
   bf16* B;
-  int n, np, c, ch;
+  int n, np, ch;
 };
 
-// Output rows of the GEMM are the 4*Ch projections interleaved in 16-row
-// blocks [a_p | a_g | a_p | a_g ... | b_p | b_g ...] (read in place through
-// the row functor, no copy), so a wave's fragments j (value) and j + 1
-// (gate) hold the same 16 channels.  Accumulator: one channel, four pairs
-// per lane per row block; two row blocks give 8 consecutive pairs -> 16-byte
-// stores into the channel-major planes.
-__global__ __launch_bounds__(512) void trimul_proj_wide_kernel(TrimulWideProjArgs a, int ncol) {
-  __shared__ __attribute__((aligned(16))) bf16 sm[kWNS * WideShape::STAGE_ELEMS];
+// Row-stationary GEMM (astat.hpp): a stage is 16 value rows and the 16 gate
+// rows of the same channels, [a_p | a_g] for the first Ch / 16 stages, then
+// [b_p | b_g].  Row block i, MFMA row m of a wave is pair 32 (i >> 1) +
+// 8 (m >> 2) + 4 (i & 1) + (m & 3) of its 64, so a lane's results of row
+// blocks 0, 1 (2, 3) are 8 consecutive pairs of one channel: the 64 pairs lie
+// in one row x (Np is a multiple of 64) and fill the channel's 128-byte line,
+// which lanes r16 and r16 ^ 1 (channels chan, chan ^ 1) store whole with the
+// streaming policy (store_line_pair).  gridDim: row tiles x csplit.
+// C = Ch = 384, N = 517: 437 -> 340 us against tiles that stage both operands
+// (256 x 128, K = 384), MFMA bound at 930 TF/s.
+template <int KT>
+__global__ __launch_bounds__(256, 2) void trimul_proj_wide_kernel(TrimulWideProjArgs a,
+                                                                  int csplit) {
+  constexpr int C = KT * 32;
+  __shared__ __attribute__((aligned(16))) bf16 sm[AstatShape<4, KT>::LDS];
+  float* mk_s = astat_row_floats<KT>(sm);
   int rt, ct;
-  wide_tile_map(blockIdx.x, ncol, rt, ct);
-  const int64_t x0 = (int64_t)rt * kWTX;
-  const int y0 = ct * kWTY;
-  const int C = a.c, CH = a.ch, np = a.np;
-  f32x4 acc[WideShape::MX][WideShape::MY];
-  // Tile row r (staged in LDS row r) is pair x0 + wide_pair_perm(r): within
-  // each 32 rows, row block 2p + b, MFMA row m is pair 8 (m >> 2) + 4 b +
-  // (m & 3), so a lane's results of row blocks 2p and 2p + 1 are 8
-  // consecutive pairs of one channel (one 16-byte store).
-  auto wide_pair_perm = [](int r) {
-    const int m = r & 15;
-    return (r & ~31) + 8 * (m >> 2) + 4 * ((r >> 4) & 1) + (m & 3);
-  };
-  gemm_nt_mainloop<kWTX, kWTY, kWWX, kWNS, false, kWKC>(
-      [&](int r) { return a.zn + (x0 + wide_pair_perm(r)) * C; },
-      [&](int r) {
-        const int R = y0 + r, side = R / (2 * CH), within = R % (2 * CH), t = within & 31;
-        const int chan = side * CH + (within >> 5) * 16 + (t & 15);
-        return (t < 16 ? a.wp : a.wg) + (size_t)chan * C;
-      },
-      C, sm, acc);
-  const int w = wave_id(), l = lane_id(), g = l >> 4, r16 = l & 15;
-  const int wx = w % kWWX, wy = w / kWWX;
-  // The wave's 64 pairs lie in one row x (np is a multiple of 64): row blocks
-  // 0, 1 give a lane pairs y + 8g .. + 7 (slot g of the channel's 128-byte
-  // line of this row), row blocks 2, 3 the pairs 32 further (slot 4 + g);
-  // lanes r16 and r16 ^ 1 (channels chan, chan ^ 1) complete each other's
-  // lines, stored whole with the streaming policy (store_line_pair).
-  static_assert(WideShape::MX == 4 && kWTX / kWWX == 64, "one 64-pair line per channel and wave");
-  const int64_t mw = x0 + wx * (kWTX / kWWX);
+  wide_tile_map(blockIdx.x, csplit, rt, ct);
+  const int CH = a.ch, np = a.np;
+  const int64_t x0 = (int64_t)rt * 256;
+  if (x0 >= (int64_t)a.n * np) return;
+  const int w = __builtin_amdgcn_readfirstlane(wave_id());
+  const int64_t mw = x0 + 64 * w;
   const int x = (int)(mw / np), yw = (int)(mw % np);
-  if (x >= a.n) return;  // rows past n * np (the last row tiles)
-  float mk[2][8];
-#pragma unroll
-  for (int hh = 0; hh < 2; ++hh)
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const int y = yw + 32 * hh + 8 * g + e;
-      mk[hh][e] = y < a.n
-                      ? (a.mask ? a.mask[(int64_t)x * a.m_s0 + (int64_t)y * a.m_s1] : 1.0f)
-                      : 0.f;
-    }
-#pragma unroll
-  for (int j = 0; j < WideShape::MY; j += 2) {
-    const int R = y0 + wy * (kWTY / WideShape::WY) + 16 * j;  // first row of the value block
-    const int side = R / (2 * CH), chan = ((R % (2 * CH)) >> 5) * 16 + r16;
-    bf16x8 v[2];
-#pragma unroll
-    for (int hh = 0; hh < 2; ++hh)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int i = 2 * hh;
-        v[hh][e] = (bf16)(mk[hh][e] * sigmoidf_(acc[i][j + 1][e]) * acc[i][j][e]);
-        v[hh][4 + e] = (bf16)(mk[hh][4 + e] * sigmoidf_(acc[i + 1][j + 1][e]) * acc[i + 1][j][e]);
-      }
-    bf16* dst = side ? a.B : a.A;
-    store_line_pair(reinterpret_cast<bf16x8*>(dst + ((size_t)chan * np + x) * np + yw),
-                    reinterpret_cast<bf16x8*>(dst + ((size_t)(chan ^ 1) * np + x) * np + yw), g,
-                    v[0], v[1]);
+  const bool live = x < a.n;
+  Frag<bf16> A[4][KT];
+  const int l = astat_lane(), g = l >> 4, r16 = l & 15;
+  if (live) {
+    const int y = yw + l;
+    mk_s[64 * w + l] =
+        y < a.n ? (a.mask ? a.mask[(int64_t)x * a.m_s0 + (int64_t)y * a.m_s1] : 1.0f) : 0.f;
   }
+  astat_load_rows<4, KT>(
+      [&](int i) {
+        return a.zn + (mw + 32 * (i >> 1) + 8 * (r16 >> 2) + 4 * (i & 1) + (r16 & 3)) * C;
+      },
+      l, A);
+  astat_rows_ready<4, KT>(A);
+  const int nst = 2 * CH / 16 / csplit, st0 = ct * nst;
+  astat_loop<KT, 2>(
+      nst, live, sm, l,
+      [&](int st) {  // LDS rows 0-15: values, 16-31: gates
+        return ((w & 2) ? a.wg : a.wp) + (size_t)((st0 + st) * 16 + 8 * (w & 1)) * C;
+      },
+      [](int r) { return r; },
+      [&](int st, const bf16* buf) __attribute__((always_inline)) {
+        f32x4 acc[4][2];
+        astat_mult<4, KT, false>(buf, l, A, acc);
+        const int ch0 = (st0 + st) * 16, side = ch0 >= CH, chan = ch0 - side * CH + r16;
+        bf16x8 v[2];
+#pragma unroll
+        for (int hh = 0; hh < 2; ++hh) {
+          float mk[8];
+          load8(mk_s + 64 * w + 32 * hh + 8 * g, mk);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int i = 2 * hh;
+            v[hh][e] = (bf16)(mk[e] * sigmoidf_(acc[i][1][e]) * acc[i][0][e]);
+            v[hh][4 + e] = (bf16)(mk[4 + e] * sigmoidf_(acc[i + 1][1][e]) * acc[i + 1][0][e]);
+          }
+        }
+        bf16* dst = (side ? a.B : a.A) + (size_t)x * np + yw;
+        const size_t plane = (size_t)np * np;
+        store_line_pair(reinterpret_cast<bf16x8*>(dst + chan * plane),
+                        reinterpret_cast<bf16x8*>(dst + (chan ^ 1) * plane), g, v[0], v[1]);
+      });
 }
 
 template <typename ZT>
@@ -1301,7 +1299,6 @@ template <typename ZT>
 int run_trimul_wide(const odde_trimul_args* a, const TrimulWs& ws, hipStream_t st) {
   const int n = a->n, C = a->c, ch = a->c_hidden, np = trimul_np(n, ODDE_BF16);
   const bool outgoing = a->outgoing != 0;
-  const int64_t vs0 = outgoing ? a->z_s0 : a->z_s1, vs1 = outgoing ? a->z_s1 : a->z_s0;
   const int64_t rows = trimul_wide_rows(n, np);
   const int row_tiles = (int)(rows / kWTX);          // a multiple of 8
   bf16* zn = static_cast<bf16*>(ws.zn);
@@ -1309,15 +1306,16 @@ int run_trimul_wide(const odde_trimul_args* a, const TrimulWs& ws, hipStream_t s
     LaunchScope ls(ODDE_K_TRIMUL_PROJ, st);
     const int lg = (int)std::min<int64_t>((int64_t)n * np / 16, 4096);
     const ZT* z = static_cast<const ZT*>(a->z);
+    const int64_t vs0 = outgoing ? a->z_s0 : a->z_s1, vs1 = outgoing ? a->z_s1 : a->z_s0;
     if (C == 128)
-      hipLaunchKernelGGL((ln_view_bf16_kernel<ZT, 128>), dim3(lg), dim3(256), 0, st, z, vs0, vs1, n, n,
-                         np, a->norm_in_weight, a->norm_in_bias, a->eps, zn);
+      hipLaunchKernelGGL((ln_view_bf16_kernel<ZT, 128>), dim3(lg), dim3(256), 0, st, z, vs0, vs1,
+                         n, n, np, a->norm_in_weight, a->norm_in_bias, a->eps, zn);
     else if (C == 256)
-      hipLaunchKernelGGL((ln_view_bf16_kernel<ZT, 256>), dim3(lg), dim3(256), 0, st, z, vs0, vs1, n, n,
-                         np, a->norm_in_weight, a->norm_in_bias, a->eps, zn);
+      hipLaunchKernelGGL((ln_view_bf16_kernel<ZT, 256>), dim3(lg), dim3(256), 0, st, z, vs0, vs1,
+                         n, n, np, a->norm_in_weight, a->norm_in_bias, a->eps, zn);
     else
-      hipLaunchKernelGGL((ln_view_bf16_kernel<ZT, 384>), dim3(lg), dim3(256), 0, st, z, vs0, vs1, n, n,
-                         np, a->norm_in_weight, a->norm_in_bias, a->eps, zn);
+      hipLaunchKernelGGL((ln_view_bf16_kernel<ZT, 384>), dim3(lg), dim3(256), 0, st, z, vs0, vs1,
+                         n, n, np, a->norm_in_weight, a->norm_in_bias, a->eps, zn);
     TrimulWideProjArgs p;
     p.zn = zn;
     p.wp = static_cast<const bf16*>(a->p_in_weight);
@@ -1327,9 +1325,19 @@ int run_trimul_wide(const odde_trimul_args* a, const TrimulWs& ws, hipStream_t s
     p.m_s1 = outgoing ? a->mask_s1 : a->mask_s0;
     p.A = static_cast<bf16*>(ws.A);
     p.B = static_cast<bf16*>(ws.B);
-    p.n = n; p.np = np; p.c = C; p.ch = ch;
-    const int ncol = 4 * ch / kWTY;
-    hipLaunchKernelGGL(trimul_proj_wide_kernel, dim3(row_tiles * ncol), dim3(512), 0, st, p, ncol);
+    p.n = n; p.np = np; p.ch = ch;
+    // projection with its LayerNorm pass, C = Ch = 384, us at split 1 / 2 / 4 /
+    // 8: N = 640 (1600 row tiles) 614 / 608 / 649 / 728, 517 (1163) 456 / 464 /
+    // 489 / 540, 300 (375) 165 / 154 / 165 / 189, 200 (200) 97 / 83 / 90 / 98,
+    // 128 (64) 81 / 52 / 38 / 38, 40 (10) 74 / 45 / 31 / 23 (16: 20)
+    const int csplit = astat_csplit(row_tiles, 2 * ch / 16, 384);
+    const dim3 pg(row_tiles * csplit);
+    if (C == 128)
+      hipLaunchKernelGGL(trimul_proj_wide_kernel<4>, pg, dim3(256), 0, st, p, csplit);
+    else if (C == 256)
+      hipLaunchKernelGGL(trimul_proj_wide_kernel<8>, pg, dim3(256), 0, st, p, csplit);
+    else
+      hipLaunchKernelGGL(trimul_proj_wide_kernel<12>, pg, dim3(256), 0, st, p, csplit);
     int rc = check_launch("trimul_proj (wide)");
     if (rc) return rc;
   }
