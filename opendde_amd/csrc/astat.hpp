@@ -191,6 +191,7 @@ __device__ __forceinline__ void astat_loop(int nst, bool live, bf16* sm, int l, 
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // own reads of stage st - 1 done
     barrier_nofence();
     if (st + 1 < nst) issue(st + 1);  // the buffer last read in stage st - 1
+    __builtin_amdgcn_sched_barrier(0);  // the loads before the stage's stores
     if (live) stage(st, sm + (st & 1) * S::STAGE);
   }
 }

@@ -304,13 +304,4 @@ __device__ __forceinline__ void gemm_nt_mainloop_pipe64_k(
   barrier_nofence();
 }
 
-// K contiguous per row: stage st at k = 64 st.
-template <int TX, int TY, int WX, bool kPairCols, typename ARow, typename BRow>
-__device__ __forceinline__ void gemm_nt_mainloop_pipe64(
-    ARow arow, BRow brow, int K, bf16* sm,
-    f32x4 (&acc)[GemmShape<TX, TY, WX, 64>::MX][GemmShape<TX, TY, WX, 64>::MY]) {
-  gemm_nt_mainloop_pipe64_k<TX, TY, WX, kPairCols>(
-      arow, brow, K / 64, [](bool, int st) { return st * 64; }, sm, acc);
-}
-
 }  // namespace odde

@@ -11,6 +11,7 @@
 // activations never touch memory.
 #include <algorithm>
 
+#include "astat.hpp"
 #include "common.hpp"
 #include "gemm.hpp"
 #include "lnpass.hpp"
@@ -976,7 +977,7 @@ __global__ __launch_bounds__(256) void transition_pair_bias_kernel(TransitionArg
   }
 }
 
-constexpr int kTwTX = 256, kTwTY = 128, kTwWX = 4, kTwNS = 3, kTwKC = 32;
+constexpr int kTwTX = 128, kTwTY = 128, kTwWX = 4, kTwNS = 3, kTwKC = 32;
 using TwShape = GemmShape<kTwTX, kTwTY, kTwWX, kTwKC>;
 
 __device__ __forceinline__ void tw_tile_map(int L, int ncol, int& rt, int& ct) {
@@ -985,123 +986,254 @@ __device__ __forceinline__ void tw_tile_map(int L, int ncol, int& rt, int& ct) {
   ct = s % ncol;
 }
 
-template <int TX, int TY = kTwTY, int KC = kTwKC>
+// Few rows: 128 x 128 tiles over the normalised rows yn.
 __global__ __launch_bounds__(512) void transition_wide_gate_kernel(const bf16* __restrict__ yn,
                                                                    const bf16* __restrict__ wa,
                                                                    const bf16* __restrict__ wb,
                                                                    bf16* __restrict__ h, int C,
                                                                    int ncol) {
-  using TwShape = GemmShape<TX, TY, kTwWX, KC>;
-  constexpr int NS = KC == 64 ? 2 : kTwNS;
-  __shared__ __attribute__((aligned(16))) bf16 sm[NS * TwShape::STAGE_ELEMS];
+  __shared__ __attribute__((aligned(16))) bf16 sm[kTwNS * TwShape::STAGE_ELEMS];
   int rt, ct;
   tw_tile_map(blockIdx.x, ncol, rt, ct);
-  const int64_t x0 = (int64_t)rt * TX;
-  const int y0 = ct * TY, HID = 4 * C;
+  const int64_t x0 = (int64_t)rt * kTwTX;
+  const int y0 = ct * kTwTY, HID = 4 * C;
   f32x4 acc[TwShape::MX][TwShape::MY];
   auto arow = [&](int r) { return yn + (x0 + r) * C; };
-  // Columns come in 32-wide groups q = R >> 5: 16 of W_a then the same 16
-  // hidden units of W_b.  With 256-wide tiles (a wave's 128 columns = 64
-  // hidden units, one 128-byte line of h per row) group q's column n is
-  // hidden unit 64 (q >> 2) + 32 ((q >> 1) & 1) + 8 (n >> 2) + 4 (q & 1) +
-  // (n & 3), so that a lane's groups 2k and 2k + 1 are 8 consecutive units;
-  // otherwise 16 (q) + n.
-  constexpr bool kLines = TY == 256;
+  // Columns come in 32-wide groups q = R >> 5: 16 hidden units' rows of W_a,
+  // then the same units' of W_b.
   auto brow = [&](int r) {
-    const int R = y0 + r, t = R & 31, q = R >> 5, nn = t & 15;
-    const int hid = kLines ? 64 * (q >> 2) + 32 * ((q >> 1) & 1) + 8 * (nn >> 2) + 4 * (q & 1) +
-                                 (nn & 3)
-                           : q * 16 + nn;
-    return (t < 16 ? wa : wb) + (size_t)hid * C;
+    const int R = y0 + r, t = R & 31;
+    return (t < 16 ? wa : wb) + (size_t)((R >> 5) * 16 + (t & 15)) * C;
   };
-  if constexpr (KC == 64)
-    gemm_nt_mainloop_pipe64<TX, TY, kTwWX, true>(arow, brow, C, sm, acc);
-  else
-    gemm_nt_mainloop<TX, TY, kTwWX, NS, true, KC>(arow, brow, C, sm, acc);
+  gemm_nt_mainloop<kTwTX, kTwTY, kTwWX, kTwNS, true, kTwKC>(arow, brow, C, sm, acc);
   const int w = wave_id(), l = lane_id(), g = l >> 4, r16 = l & 15;
   const int wx = w % kTwWX, wy = w / kTwWX;
 #pragma unroll
   for (int i = 0; i < TwShape::MX; ++i) {
-    const int64_t m = x0 + wx * (TX / kTwWX) + 16 * i + r16;
-    if constexpr (kLines) {
-      // hidden units 64 (2 ct + wy) + 8g .. + 7 (slot g of row m's line) from
-      // groups 0, 1 of the wave, the same + 32 (slot 4 + g) from groups 2, 3;
-      // rows m and m ^ 1 (lanes r16, r16 ^ 1) complete each other's lines
-      static_assert(TwShape::MY == 8, "four column groups per wave");
-      bf16x8 v[2];
+    const int64_t m = x0 + wx * (kTwTX / kTwWX) + 16 * i + r16;
 #pragma unroll
-      for (int hh = 0; hh < 2; ++hh)
+    for (int j = 0; j < TwShape::MY; j += 2) {
+      const int hid = ((y0 + wy * (kTwTY / TwShape::WY) + 16 * j) >> 5) * 16 + 4 * g;
+      bf16x4 v;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int j = 4 * hh;
-          v[hh][e] = (bf16)(siluf_(acc[i][j][e]) * acc[i][j + 1][e]);
-          v[hh][4 + e] = (bf16)(siluf_(acc[i][j + 2][e]) * acc[i][j + 3][e]);
-        }
-      const int hb = (y0 + wy * (TY / TwShape::WY)) / 2;  // the wave's first hidden unit
-      store_line_pair(reinterpret_cast<bf16x8*>(h + m * HID + hb),
-                      reinterpret_cast<bf16x8*>(h + (m ^ 1) * HID + hb), g, v[0], v[1]);
-    } else {
-#pragma unroll
-      for (int j = 0; j < TwShape::MY; j += 2) {
-        const int hid = ((y0 + wy * (TY / TwShape::WY) + 16 * j) >> 5) * 16 + 4 * g;
-        bf16x4 v;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = (bf16)(siluf_(acc[i][j][e]) * acc[i][j + 1][e]);
-        *reinterpret_cast<bf16x4*>(h + m * HID + hid) = v;
-      }
+      for (int e = 0; e < 4; ++e) v[e] = (bf16)(siluf_(acc[i][j][e]) * acc[i][j + 1][e]);
+      *reinterpret_cast<bf16x4*>(h + m * HID + hid) = v;
     }
   }
 }
 
-// kSplit > 1: workgroup column ks of the grid (blockIdx.y) takes hidden
-// units [ks HID / kSplit, (ks + 1) HID / kSplit) and writes its fp32 partial
-// sums to part[ks][m][c] (rows of the padded tile range); the residual is
-// added by transition_wide_reduce_kernel, which sums the partials in order.
-template <typename ZT, int TX, int kSplit>
+// The gate GEMM of many rows, row-stationary (astat.hpp) with the LayerNorm
+// fused into the row loads (16 MB rows a wave): a stage is 16 hidden units, LDS rows 0-15 their
+// W_a rows, 16-31 their W_b rows.  The hidden rows go out in blocks of 64 rows
+// x 16 units: h[row / 64][unit / 16][row % 64][unit % 16], so that a wave's
+// four stores of a stage are 2 KiB on end and the output GEMM reads its
+// fragments 512 bytes at a time.  262144 rows: LayerNorm pass and 256 x 256
+// tiles 876 us, now 660 (940 TF/s with the LayerNorm; MFMA busy 56% of the
+// cycles, at 2.0 GHz under this load).
+template <int MB, int KT, typename ZT>
+__global__ __launch_bounds__(256, 2) void transition_rows_gate_kernel(
+    const ZT* __restrict__ x, const float* __restrict__ ln_w, const float* __restrict__ ln_b,
+    float eps, const bf16* __restrict__ wa, const bf16* __restrict__ wb, bf16* __restrict__ h,
+    int64_t rows, int csplit) {
+  constexpr int C = KT * 32, HB = 4 * C / 16;  // hidden blocks of 16 units
+  __shared__ __attribute__((aligned(16))) bf16 sm[AstatShape<MB, KT>::LDS];
+  int rt, ct;
+  tw_tile_map(blockIdx.x, csplit, rt, ct);
+  const int64_t x0 = (int64_t)rt * (64 * MB);
+  if (x0 >= rows) return;
+  const int w = __builtin_amdgcn_readfirstlane(wave_id());
+  const int64_t mw = x0 + 16 * MB * w;
+  const bool live = mw < rows;
+  Frag<bf16> A[MB][KT];
+#pragma unroll
+  for (int i = 0; i < MB; ++i) {
+    const int64_t m = mw + 16 * i + (lane_id() & 15);
+    const bool valid = m < rows;
+    astat_ln_rows<MB == 4, KT>(x + (valid ? m : 0) * C, valid, ln_w, ln_b, eps, A[i]);
+  }
+  const int l = astat_lane(), g = l >> 4, r16 = l & 15;
+  astat_rows_ready<MB, KT>(A);
+  const int nst = HB / csplit, st0 = ct * nst;
+  const bf16* W = ((w & 2) ? wb : wa) + (size_t)(st0 * 16 + 8 * (w & 1)) * C;
+  bf16* hw = h + (((mw >> 6) * HB + st0) * 64 + (mw & 63)) * 16;
+  const int lo = r16 * 16 + 4 * g;
+  astat_loop<KT, MB>(
+      nst, live, sm, l, [&](int st) { return W + (size_t)st * 16 * C; },
+      [](int r) { return r; },
+      [&](int st, const bf16* buf) __attribute__((always_inline)) {
+        f32x4 acc[MB][2];
+        astat_mult<MB, KT, true>(buf, l, A, acc);
+        bf16* d = hw + (size_t)st * 1024;
+#pragma unroll
+        for (int i = 0; i < MB; ++i) {
+          bf16x4 v;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] = (bf16)(siluf_(acc[i][0][e]) * acc[i][1][e]);
+          *reinterpret_cast<bf16x4*>(d + lo + i * 256) = v;
+        }
+      });
+}
+
+// The output GEMM of many rows over the blocked hidden rows: K = 4 C, N = C.
+// A workgroup of 4 waves owns 128 rows x 192 columns, a wave 64 x 96; two
+// workgroups per CU, so one's epilogue and first loads run under the other's
+// MFMAs.  The hidden fragments come straight from global memory into
+// registers, two stages of 64 k ahead; only the weights go through LDS (three
+// stage buffers), which halves the LDS cycles per MFMA against staging both.
+// 262144 rows: 435 us as 256 x 128 tiles of both operands, now 415 (745 TF/s);
+// one stage ahead instead of two 425.
+constexpr int kToRows = 128, kToCols = 192;
+template <typename ZT, int C>
+__global__ __launch_bounds__(256, 2) void transition_rows_out_kernel(
+    const bf16* __restrict__ h, const bf16* __restrict__ wo, const ZT* x, ZT* out, int64_t rows,
+    int add) {
+  constexpr int HID = 4 * C, HB = HID / 16, NST = HID / 64;
+  constexpr int STAGE = kToCols * 64, NCOL = C / kToCols;
+  static_assert(C % kToCols == 0 && NST % 3 == 0, "whole column tiles, stages in threes");
+  __shared__ __attribute__((aligned(16))) bf16 sm[3 * STAGE];
+  int rt, ct;
+  tw_tile_map(blockIdx.x, NCOL, rt, ct);
+  const int64_t x0 = (int64_t)rt * kToRows;
+  if (x0 >= rows) return;
+  const int w = __builtin_amdgcn_readfirstlane(wave_id()), l = lane_id(), g = l >> 4, r16 = l & 15;
+  const int wx = w & 1, wy = w >> 1;
+  const int y0 = ct * kToCols;
+  const int64_t mw = x0 + 64 * wx;
+  // A fragment (row block i, k step t): k block 2 t + g / 2, units 8 (g & 1) ..
+  const bf16* hw = h + (mw >> 6) * HB * 1024;
+  const int alane = (g >> 1) * 1024 + r16 * 16 + (g & 1) * 8;
+  // weight rows 48 w .. 48 w + 47 of the tile: six loads of 8 rows x 64 k
+  const int lr = l >> 3;
+  const bf16* wsrc = wo + (size_t)(y0 + 48 * w) * HID;
+  const uint32_t voff = (uint32_t)(lr * HID + (((l & 7) ^ lr) * 8)) * (uint32_t)sizeof(bf16);
+  auto issue = [&](auto slot, int st) {
+    bf16* dst = sm + decltype(slot)::value * STAGE + 48 * w * 64;
+#pragma unroll
+    for (int k = 0; k < 6; ++k)
+      buffer_load_lds16(wsrc, 48 * HID * (uint32_t)sizeof(bf16), dst + k * 512, voff,
+                        (uint32_t)(k * 8 * HID + st * 64) * (uint32_t)sizeof(bf16));
+  };
+  Frag<bf16> A[3][2][4];  // [stage % 3][k step][row block]
+  auto load_a = [&](auto slot, int st) {
+    constexpr int p = decltype(slot)::value;
+    const bf16* src = hw + (size_t)st * 4096;
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) A[p][t][i].load(src + t * 2048 + i * 256 + alane);
+  };
+  f32x4 acc[4][6];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 6; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int b0 = (96 * wy + r16) * 64 + ((g ^ (r16 & 7)) * 8);
+  const int b1 = (96 * wy + r16) * 64 + (((4 + g) ^ (r16 & 7)) * 8);
+  auto mult = [&](auto slot) {
+    constexpr int p = decltype(slot)::value;
+    const bf16* base = sm + p * STAGE;
+    Frag<bf16> b[3];
+    auto read = [&](int u) {  // fragment u = (k step u / 6, column block u % 6)
+      b[u % 3].load(base + (u < 6 ? b0 : b1) + (u % 6) * (16 * 64));
+    };
+    read(0);
+    read(1);
+#pragma unroll
+    for (int u = 0; u < 12; ++u) {
+      if (u + 2 < 12) read(u + 2);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) mma(acc[i][u % 6], b[u % 3], A[p][u / 6][i]);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+#pragma unroll
+    for (int u = 0; u < 10; ++u) {
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x008, 8, 0);
+  };
+  // stage st: slot st % 3 of the weights (LDS) and of the rows (registers)
+  auto stage = [&](auto slot, auto ahead, int st) {
+    // this wave's weights of stage st landed: younger are the rows of stage st
+    // and the weights and rows of stage st + 1 (8 + 6 + 8)
+    asm volatile("s_waitcnt vmcnt(22)" ::: "memory");
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // own reads of stage st - 1 done
+    barrier_nofence();
+    // stage st + 2 into the slots of stage st - 1; past the end stage NST - 1
+    // again, never used (a branch here would make the compiler wait for these
+    // loads before it uses the rows of stage st)
+    issue(ahead, min(st + 2, NST - 1));
+    __builtin_amdgcn_sched_barrier(0);  // in this order: the wait above counts on it
+    load_a(ahead, min(st + 2, NST - 1));
+    __builtin_amdgcn_sched_barrier(0);
+    mult(slot);
+  };
+  using P0 = std::integral_constant<int, 0>;
+  using P1 = std::integral_constant<int, 1>;
+  using P2 = std::integral_constant<int, 2>;
+  issue(P0{}, 0);
+  __builtin_amdgcn_sched_barrier(0);
+  load_a(P0{}, 0);
+  __builtin_amdgcn_sched_barrier(0);
+  issue(P1{}, 1);
+  __builtin_amdgcn_sched_barrier(0);
+  load_a(P1{}, 1);
+  __builtin_amdgcn_sched_barrier(0);
+  for (int st = 0; st < NST; st += 3) {
+    stage(P0{}, P2{}, st);
+    stage(P1{}, P0{}, st + 1);
+    stage(P2{}, P1{}, st + 2);
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no load into LDS outlives the wave
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    // rows m and m ^ 1 (lanes r16, r16 ^ 1) complete each other's lines
+    const int64_t m = mw + 16 * i + r16;
+    const bool ok = m < rows, pok = (m ^ 1) < rows;
+    const int cw = y0 + 96 * wy;
+    float r[6][4];
+#pragma unroll
+    for (int j = 0; j < 6; ++j) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) r[j][e] = 0.f;
+      if (add && ok) load4(x + m * C + cw + 16 * j + 4 * g, r[j]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) r[j][e] += acc[i][j][e];
+    }
+    store_row_blocks<ZT>(out + m * C, out + (m ^ 1) * C, cw, r, ok, pok);
+  }
+}
+
+// Workgroup column ks of the grid (blockIdx.y) takes hidden units [ks HID /
+// kSplit, (ks + 1) HID / kSplit) and writes its fp32 partial sums to
+// part[ks][m][c] (rows of the padded tile range); transition_wide_reduce_kernel
+// sums the partials in order and adds the residual.
+template <int kSplit>
 __global__ __launch_bounds__(512) void transition_wide_out_kernel(const bf16* __restrict__ h,
                                                                   const bf16* __restrict__ wo,
-                                                                  const ZT* x, ZT* out,
                                                                   float* __restrict__ part,
                                                                   int64_t rows, int64_t mp,
-                                                                  int C, int add, int ncol) {
-  using TwShape = GemmShape<TX, kTwTY, kTwWX, kTwKC>;
+                                                                  int C, int ncol) {
   __shared__ __attribute__((aligned(16))) bf16 sm[kTwNS * TwShape::STAGE_ELEMS];
   int rt, ct;
   tw_tile_map(blockIdx.x, ncol, rt, ct);
-  const int64_t x0 = (int64_t)rt * TX;
+  const int64_t x0 = (int64_t)rt * kTwTX;
   const int y0 = ct * kTwTY, HID = 4 * C, KS = HID / kSplit, k0 = (int)blockIdx.y * KS;
   f32x4 acc[TwShape::MX][TwShape::MY];
-  gemm_nt_mainloop<TX, kTwTY, kTwWX, kTwNS, true, kTwKC>(
+  gemm_nt_mainloop<kTwTX, kTwTY, kTwWX, kTwNS, true, kTwKC>(
       [&](int r) { return h + (x0 + r) * HID + k0; },
       [&](int r) { return wo + (size_t)(y0 + r) * HID + k0; }, KS, sm, acc);
   const int w = wave_id(), l = lane_id(), g = l >> 4, r16 = l & 15;
   const int wx = w % kTwWX, wy = w / kTwWX;
 #pragma unroll
   for (int i = 0; i < TwShape::MX; ++i) {
-    const int64_t m = x0 + wx * (TX / kTwWX) + 16 * i + r16;
-    if constexpr (kSplit > 1) {
-      if (m >= rows) continue;
+    const int64_t m = x0 + wx * (kTwTX / kTwWX) + 16 * i + r16;
+    if (m >= rows) continue;
 #pragma unroll
-      for (int j = 0; j < TwShape::MY; ++j) {
-        const int c0 = y0 + wy * (kTwTY / TwShape::WY) + 16 * j + 4 * g;
-        store4(part + ((int64_t)blockIdx.y * mp + m) * C + c0, acc[i][j][0], acc[i][j][1],
-               acc[i][j][2], acc[i][j][3]);
-      }
-    } else {
-      // rows m and m ^ 1 (lanes r16, r16 ^ 1) complete each other's lines
-      const bool ok = m < rows, pok = (m ^ 1) < rows;
-      float r[TwShape::MY][4];
-#pragma unroll
-      for (int j = 0; j < TwShape::MY; ++j) {
-        const int c0 = y0 + wy * (kTwTY / TwShape::WY) + 16 * j + 4 * g;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) r[j][e] = 0.f;
-        if (add && ok) load4(x + m * C + c0, r[j]);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) r[j][e] += acc[i][j][e];
-      }
-      store_row_blocks<ZT>(out + m * C, out + (m ^ 1) * C, y0 + wy * (kTwTY / TwShape::WY), r,
-                           ok, pok);
+    for (int j = 0; j < TwShape::MY; ++j) {
+      const int c0 = y0 + wy * (kTwTY / TwShape::WY) + 16 * j + 4 * g;
+      store4(part + ((int64_t)blockIdx.y * mp + m) * C + c0, acc[i][j][0], acc[i][j][1],
+             acc[i][j][2], acc[i][j][3]);
     }
   }
 }
@@ -1142,15 +1274,17 @@ void launch_tr(const TransitionArgs<ZT, CT>& p, hipStream_t st) {
 }
 
 bool transition_wide(int c, int nf, int dt) { return dt == ODDE_BF16 && c == 384 && nf == 4; }
-// Up to kTwSmallRows rows (the single track) the GEMMs take 128-row tiles
-// and the output GEMM splits the hidden dimension kTwSplit ways, so that a
-// few hundred rows still fill the GPU; tile rows are padded to whole groups
-// of 8 row tiles (tw_tile_map).
-constexpr int64_t kTwSmallRows = 16384;
+// Up to kTwSmallRows rows (the single track) a LayerNorm pass and GEMMs of
+// 128-row tiles, the output GEMM with the hidden dimension split kTwSplit
+// ways, so that a few hundred rows still fill the GPU; above, the
+// row-stationary gate and the output GEMM over its blocked hidden rows (us,
+// this / those: 2048 rows 33 / 42, 4096 46 / 46, 6400 68 / 57, 16384 130 / 79).
+// Rows are padded to whole groups of 8 row tiles (tw_tile_map).
+constexpr int64_t kTwSmallRows = 4096;
 constexpr int kTwSplit = 4;
 bool transition_wide_small(int64_t rows) { return rows <= kTwSmallRows; }
 int64_t transition_wide_rows(int64_t rows) {
-  const int64_t q = transition_wide_small(rows) ? 8 * 128 : 8 * kTwTX;
+  const int64_t q = transition_wide_small(rows) ? 8 * 128 : 8 * 256;
   return (rows + q - 1) / q * q;
 }
 // fp32 arithmetic with few rows (fewer than 512 blocks of 16): the hidden
@@ -1188,48 +1322,57 @@ uint64_t transition_ws_bytes(const odde_transition_args* a) {
   // normalised rows [Mp][C] and hidden activations [Mp][4C], bf16; with the
   // split output GEMM its fp32 partial sums [kTwSplit][Mp][C]
   const uint64_t mp = (uint64_t)transition_wide_rows(a->rows);
-  const uint64_t part = transition_wide_small(a->rows) ? (uint64_t)kTwSplit * mp * a->c * 4 : 0;
-  return mp * 5 * a->c * 2 + part + 256;
+  // hidden rows; the small form's normalised rows and partial sums
+  const uint64_t small =
+      transition_wide_small(a->rows) ? mp * a->c * 2 + (uint64_t)kTwSplit * mp * a->c * 4 : 0;
+  return mp * 4 * a->c * 2 + small + 256;
 }
 
 template <typename ZT>
 int run_transition_wide(const odde_transition_args* a, hipStream_t st) {
   const int C = a->c;
   const int64_t rows = a->rows, mp = transition_wide_rows(rows);
-  bf16* yn = static_cast<bf16*>(a->workspace);
-  bf16* h = yn + mp * C;
+  bf16* h = static_cast<bf16*>(a->workspace);
   LaunchScope ls(ODDE_K_TRANSITION, st);
-  const int lg = (int)std::min<int64_t>((rows + 15) / 16, 4096);
-  // rows as one view row of length `rows` (x = 0, y = row)
-  hipLaunchKernelGGL((ln_view_bf16_kernel<ZT, 384>), dim3(lg), dim3(256), 0, st,
-                     static_cast<const ZT*>(a->x), (int64_t)0, (int64_t)C, (int)rows, 1,
-                     (int)rows, a->ln_w, a->ln_b, a->eps, yn);
-  const int ncol1 = 8 * C / kTwTY, ncol2 = C / kTwTY;
   const bf16* wa = static_cast<const bf16*>(a->w_a);
   const bf16* wb = static_cast<const bf16*>(a->w_b);
   const bf16* wo = static_cast<const bf16*>(a->w_o);
   const ZT* x = static_cast<const ZT*>(a->x);
   ZT* out = static_cast<ZT*>(a->out);
   if (transition_wide_small(rows)) {
-    const int row_tiles = (int)(mp / 128);
-    float* part = reinterpret_cast<float*>(h + mp * 4 * C);
-    hipLaunchKernelGGL(transition_wide_gate_kernel<128>, dim3(row_tiles * ncol1), dim3(512), 0, st,
+    const int row_tiles = (int)(mp / kTwTX), ncol1 = 8 * C / kTwTY, ncol2 = C / kTwTY;
+    bf16* yn = h + mp * 4 * C;
+    const int lg = (int)std::min<int64_t>((rows + 15) / 16, 4096);
+    // rows as one view row of length `rows` (x = 0, y = row)
+    hipLaunchKernelGGL((ln_view_bf16_kernel<ZT, 384>), dim3(lg), dim3(256), 0, st, x, (int64_t)0,
+                       (int64_t)C, (int)rows, 1, (int)rows, a->ln_w, a->ln_b, a->eps, yn);
+    float* part = reinterpret_cast<float*>(yn + mp * C);
+    hipLaunchKernelGGL(transition_wide_gate_kernel, dim3(row_tiles * ncol1), dim3(512), 0, st,
                        yn, wa, wb, h, C, ncol1);
-    hipLaunchKernelGGL((transition_wide_out_kernel<ZT, 128, kTwSplit>),
-                       dim3(row_tiles * ncol2, kTwSplit), dim3(512), 0, st, h, wo, x, out, part,
-                       rows, mp, C, a->add_residual, ncol2);
+    hipLaunchKernelGGL(transition_wide_out_kernel<kTwSplit>, dim3(row_tiles * ncol2, kTwSplit),
+                       dim3(512), 0, st, h, wo, part, rows, mp, C, ncol2);
     const int rg = (int)std::min<int64_t>((rows * C / 4 + 255) / 256, 2048);
     hipLaunchKernelGGL((transition_wide_reduce_kernel<ZT, kTwSplit>), dim3(rg), dim3(256), 0, st,
                        part, x, out, rows, mp, C, a->add_residual);
   } else {
-    // the gate GEMM (N = 8C): 256 x 256 tiles, 64-k pipelined stages (each
-    // wave 64 x 128, fewer LDS bytes per MFMA than 256 x 128 tiles)
-    const int row_tiles = (int)(mp / kTwTX), ncol1w = 8 * C / 256;
-    hipLaunchKernelGGL((transition_wide_gate_kernel<kTwTX, 256, 64>), dim3(row_tiles * ncol1w),
-                       dim3(512), 0, st, yn, wa, wb, h, C, ncol1w);
-    hipLaunchKernelGGL((transition_wide_out_kernel<ZT, kTwTX, 1>), dim3(row_tiles * ncol2),
-                       dim3(512), 0, st, h, wo, x, out, nullptr, rows, mp, C, a->add_residual,
-                       ncol2);
+    // 32 rows a wave up to 90000 rows, 64 above: the LayerNorm of a wave's rows
+    // runs before its first MFMA, and with 64 the grid of a middling call has
+    // too few waves to hide it.  Whole transition, us, 32 / 64 rows: 10000 rows
+    // 67 / 82, 16384 79 / 88, 40000 176 / 199, 65536 250 / 264, 90000 405 / 401.
+    // The column split at 1 / 2 / 4 / 8, 32 rows: 10000 rows (80 row tiles) 106 /
+    // 74 / 68 / 75, 16384 (128) 111 / 79 / 78 / 90, 40000 (320) 176 / 179 / 183 /
+    // 220.
+    const bool mb2 = rows <= 90000;
+    const int gt = (int)(mp / (mb2 ? 128 : 256)), csplit = astat_csplit(gt, 4 * C / 16, 256);
+    if (mb2)
+      hipLaunchKernelGGL((transition_rows_gate_kernel<2, 12, ZT>), dim3(gt * csplit), dim3(256), 0,
+                         st, x, a->ln_w, a->ln_b, a->eps, wa, wb, h, rows, csplit);
+    else
+      hipLaunchKernelGGL((transition_rows_gate_kernel<4, 12, ZT>), dim3(gt * csplit), dim3(256), 0,
+                         st, x, a->ln_w, a->ln_b, a->eps, wa, wb, h, rows, csplit);
+    const int ot = (int)(mp / kToRows) * (C / kToCols);
+    hipLaunchKernelGGL((transition_rows_out_kernel<ZT, 384>), dim3(ot), dim3(256), 0, st, h, wo, x,
+                       out, rows, a->add_residual);
   }
   if (a->pb_heads) {
     TransitionArgs<ZT, bf16> p;

@@ -101,3 +101,19 @@ def test_multiplication_plane_sizes(n, c, outgoing):
     assert_bf16(run(True), exp, f"planes bf16 n={n} c={c} out={outgoing}")
     if c == 64:
         assert_fp32(run(False), exp, f"planes n={n} c={c} out={outgoing}")
+
+
+@pytest.mark.parametrize("rows", [4095, 4097, 16417, 90001])
+@pytest.mark.parametrize("inplace", [False, True])
+def test_transition_rows_c384(rows, inplace):
+    """The wide transition's forms by row count (tiles up to 4096 rows, then 32
+    and from 90001 rows 64 rows a wave), with rows that end inside a wave."""
+    from opendde_amd.pairformer import Transition
+    say(f"[gpu] transition rows={rows} inplace={inplace}")
+    mod = seeded(Transition(384, 4), rows, 0.04)
+    x = torch.randn(rows, 384, generator=torch.Generator().manual_seed(rows))
+    exp = ref.transition(x, params_of(mod))
+    mod, xg = mod.to(DEV), x.to(DEV)
+    with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16):
+        got = mod.hip_apply(xg, out=xg, add_residual=True) if inplace else mod.hip_apply(xg)
+    assert_bf16(got.cpu() - x if inplace else got, exp, f"transition rows={rows} inplace={inplace}")
