@@ -452,18 +452,19 @@ inline void launch_contract(const ContractArgs<bf16>& k, hipStream_t st) {
                          dim3(512), 0, st, k);
   }
 }
-// fp32: 64 x 64 tiles fit every Np and give four times the workgroups (Np 128:
-// 12.1 us against 17.6 with 128 x 128, 384: 143 / 147; N = 300 89 us, against
-// 163 over planes rounded up to 128); 128 x 128 reads each operand half as
-// often from L2 and is ahead from Np = 512 (297 / 315, 640: 575 / 590).
+// fp32: 64 x 64 tiles fit every Np and give four times the workgroups (four per
+// CU, against two); 128 x 128 reads each operand half as often from L2 and
+// multiplies some 5% faster, so it is taken from Np = 512 unless its last round
+// of workgroups leaves over a tenth more of the chip idle.  us, 64 / 128, Ch =
+// 128: Np 128 12.1 / 17.6, 384 143 / 147, 512 315 / 297, 640 590 / 575; Ch = 64,
+// 640: 295 / 330.  N = 300 89 us, against 163 over planes rounded up to 128.
 inline void launch_contract(const ContractArgs<float>& k, hipStream_t st) {
-  const int np = k.np;
-  if (np % 128 == 0 && np >= 512) {
-    hipLaunchKernelGGL((trimul_contract_f32_kernel<128>), dim3((np / 128) * (np / 128) * k.ch),
-                       dim3(256), 0, st, k);
+  const int np = k.np, t64 = (np / 64) * (np / 64) * k.ch, t128 = (np / 128) * (np / 128) * k.ch;
+  const double f64 = (double)t64 / round_up(t64, 1024), f128 = (double)t128 / round_up(t128, 512);
+  if (np % 128 == 0 && np >= 512 && 1.1 * f128 >= f64) {
+    hipLaunchKernelGGL((trimul_contract_f32_kernel<128>), dim3(t128), dim3(256), 0, st, k);
   } else {
-    hipLaunchKernelGGL((trimul_contract_f32_kernel<64>), dim3((np / 64) * (np / 64) * k.ch),
-                       dim3(256), 0, st, k);
+    hipLaunchKernelGGL((trimul_contract_f32_kernel<64>), dim3(t64), dim3(256), 0, st, k);
   }
 }
 
@@ -1438,12 +1439,14 @@ void launch_tp(const TrimulProjArgs<ZT, CT>& p, hipStream_t st) {
   }
   if (kX3Out || (kRB > 1 && p.n > 128)) {
     const int rows = (p.n + kRB - 1) / kRB;
-    dim3 grid(p.np / 64, rows, proj_split((int64_t)(p.np / 64) * rows, p.ch / 16));
+    dim3 grid(p.np / 64, rows, proj_split((int64_t)(p.np / 64) * (p.np / kRB), p.ch / 16));
     hipLaunchKernelGGL((trimul_proj_kernel<ZT, CT, kC, kRB, kX3Out, kX3Mul>), grid, dim3(256), 0,
                        st, p);
     return;
   }
-  dim3 grid(p.np / 64, p.n, proj_split((int64_t)(p.np / 64) * p.n, p.ch / 16));
+  // the split by Np: a few rows short of it must not double the splits, each
+  // of which normalises the rows again
+  dim3 grid(p.np / 64, p.n, proj_split((int64_t)(p.np / 64) * p.np, p.ch / 16));
   hipLaunchKernelGGL((trimul_proj_kernel<ZT, CT, kC, 1, false, kX3Mul>), grid, dim3(256), 0, st, p);
 }
 template <typename ZT, int kC>
