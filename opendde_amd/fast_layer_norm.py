@@ -21,6 +21,7 @@ arithmetic runs in ``libopendde_amd.so`` (``odde_layer_norm_fwd`` /
 
 from __future__ import annotations
 
+import contextlib
 import ctypes
 from typing import List, Optional, Sequence, Tuple
 
@@ -78,12 +79,20 @@ def _param(p: Optional[torch.Tensor], input: torch.Tensor, n2: int, name: str):
     return p.contiguous()
 
 
-def _ptr(t: Optional[torch.Tensor]) -> ctypes.c_void_p:
-    return ctypes.c_void_p(t.data_ptr() if t is not None else 0)
+def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
+    return t.data_ptr() if t is not None else None
 
 
-def _stream(device: torch.device) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+def _stream(device: torch.device) -> int:
+    return torch._C._cuda_getCurrentRawStream(device.index)
+
+
+def _device_guard(device: torch.device):
+    """The library launches on the current device: switch to ``device`` where
+    it is another one."""
+    if torch.cuda.current_device() == device.index:
+        return contextlib.nullcontext()
+    return torch.cuda.device(device)
 
 
 def layer_norm_affine(input: torch.Tensor, normalized_shape, gamma: Optional[torch.Tensor],
@@ -103,7 +112,7 @@ def layer_norm_affine(input: torch.Tensor, normalized_shape, gamma: Optional[tor
     a.x, a.gamma, a.beta = _ptr(input), _ptr(gamma), _ptr(beta)
     a.out, a.mean, a.invvar = _ptr(output), _ptr(mean), _ptr(invvar)
     lib = _lib.load()
-    with torch.cuda.device(input.device):
+    with _device_guard(input.device):
         _lib.check(lib.odde_layer_norm_fwd(ctypes.byref(a), _stream(input.device)),
                    "odde_layer_norm_fwd")
     return [output, mean, invvar]
@@ -145,7 +154,7 @@ def layer_norm_gradient_affine(dout: torch.Tensor, mean: torch.Tensor, invvar: t
         # torch's caching allocator returns 256-byte aligned blocks
         ws = torch.empty(max(int(nb.value), 256), dtype=torch.uint8, device=input.device)
         a.workspace, a.workspace_bytes = _ptr(ws), ws.numel()
-    with torch.cuda.device(input.device):
+    with _device_guard(input.device):
         _lib.check(lib.odde_layer_norm_bwd(ctypes.byref(a), _stream(input.device)),
                    "odde_layer_norm_bwd")
     return [grad_input, grad_gamma, grad_beta]

@@ -43,12 +43,14 @@ def autocast_compute_dtype(t: torch.Tensor) -> torch.dtype:
     return torch.float32
 
 
-def _ptr(t: Optional[torch.Tensor]):
-    return ctypes.c_void_p(t.data_ptr()) if t is not None else ctypes.c_void_p(0)
+def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
+    return t.data_ptr() if t is not None else None
 
 
-def _stream(device: torch.device) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+def _stream(device: torch.device) -> int:
+    # the raw handle of the current stream (torch.cuda.current_stream builds a
+    # Stream object for it: 2 us of a small call's 55)
+    return torch._C._cuda_getCurrentRawStream(device.index)
 
 
 def _require_gpu(*ts: torch.Tensor) -> None:
@@ -75,6 +77,8 @@ def pair_layout_ok(t: torch.Tensor) -> bool:
         return False
     if t.numel() == 0:
         return True
+    if t.dim() == 3:
+        return (t.data_ptr() | (t.stride(0) | t.stride(1)) * t.element_size()) & 15 == 0
     try:
         v = t.view((-1,) + tuple(t.shape[-3:]))
     except RuntimeError:
@@ -97,6 +101,18 @@ def _batch_view(t: torch.Tensor, name: str) -> Tuple[torch.Tensor, int, int]:
     except RuntimeError:
         raise ValueError(f"{name}'s leading dims must collapse to one batch stride") from None
     return v, v.shape[0], v.stride(0) if v.shape[0] > 1 else 0
+
+
+def _pair_strides(t: torch.Tensor, name: str) -> Tuple[int, int, int, int]:
+    """(batch count, batch stride, row stride, column stride) of ``t``
+    [*, N, N, C], in elements (:func:`_batch_view` without the view for a
+    tensor that has no leading dims)."""
+    if t.dim() == 3:
+        _pair_view_ok(t, name)
+        st = t.stride()
+        return 1, 0, st[0], st[1]
+    v, b, sb = _batch_view(t, name)
+    return b, sb, v.stride(1) if b else 0, v.stride(2) if b else 0
 
 
 # Converted weights are cached per source tensor *object* (held by weak
@@ -138,7 +154,11 @@ def cache_size() -> int:
 
 def prepared(t: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
     """``t`` as a contiguous ``dtype`` tensor, converted once per version."""
-    return _cached((id(t), dtype), (t,), lambda: t.detach().to(dtype).contiguous())
+    key = (id(t), dtype)
+    ent = _wcache.get(key)
+    if ent is not None and ent[0][0]() is t and ent[1][0] == t._version:
+        return ent[2]  # _cached's hit, without its loops: a module call looks up 8 to 11
+    return _cached(key, (t,), lambda: t.detach().to(dtype).contiguous())
 
 
 def prepared_cat(ts, dtype: torch.dtype) -> torch.Tensor:
@@ -167,6 +187,16 @@ def _mask_view(mask: Optional[torch.Tensor], lead: Tuple[int, ...], n: int,
         raise ValueError(f"mask {tuple(mask.shape)} does not broadcast to z's leading dims "
                          f"{tuple(lead)}") from None
     return m, m.stride(1), m.stride(2), m.stride(0) if m.shape[0] > 1 else 0
+
+
+def _mask_args(mask: Optional[torch.Tensor], z: torch.Tensor,
+               n: int) -> Tuple[Optional[torch.Tensor], int, int, int]:
+    """:func:`_mask_view` for z, without the views where the mask is z's
+    [N, N] in float32 already."""
+    if (mask is not None and z.dim() == 3 and mask.dim() == 2 and mask.dtype == torch.float32
+            and mask.shape[0] == n and mask.shape[1] == n and mask.device == z.device):
+        return mask, mask.stride(0), mask.stride(1), 0
+    return _mask_view(mask, z.shape[:-3], n, z.device)
 
 
 # ---------------------------------------------------------------------------
@@ -260,7 +290,7 @@ def triangle_attention(z: torch.Tensor, mask: Optional[torch.Tensor], *, ln_w, l
     are true fp32.
     """
     _require_gpu(z, mask)
-    zb, nbatch, z_sb = _batch_view(z, "z")
+    nbatch, z_sb, zs0, zs1 = _pair_strides(z, "z")
     n, c = z.shape[-3], z.shape[-1]
     if c not in SUPPORTED_CHANNELS or heads * HEAD_DIM not in SUPPORTED_CHANNELS:
         raise NotImplementedError(
@@ -275,12 +305,10 @@ def triangle_attention(z: torch.Tensor, mask: Optional[torch.Tensor], *, ln_w, l
         out = torch.empty_like(z, memory_format=torch.contiguous_format)
     if out.dtype != z.dtype or out.shape != z.shape:
         raise ValueError("out must match z in shape and dtype")
-    ob, _, o_sb = _batch_view(out, "out")
-    m, ms0, ms1, m_sb = _mask_view(mask, z.shape[:-3], n, z.device)
+    _, o_sb, os0, os1 = _pair_strides(out, "out")
+    m, ms0, ms1, m_sb = _mask_args(mask, z, n)
     if z.numel() == 0:
         return out
-    zs0, zs1 = zb.stride(1), zb.stride(2)
-    os0, os1 = ob.stride(1), ob.stride(2)
     if not starting:
         zs0, zs1, ms0, ms1, os0, os1 = zs1, zs0, ms1, ms0, os1, os0
     lnw = prepared(ln_w, torch.float32)
@@ -326,7 +354,7 @@ def triangle_multiplication(z: torch.Tensor, mask: Optional[torch.Tensor], *, ou
     the projections and the output always, the contraction where Np is a
     multiple of 256 (true fp32 products otherwise)."""
     _require_gpu(z, mask)
-    zb, nbatch, z_sb = _batch_view(z, "z")
+    nbatch, z_sb, zs0, zs1 = _pair_strides(z, "z")
     n, c = z.shape[-3], z.shape[-1]
     ch = p_in_weight.shape[0] // 2
     if c not in SUPPORTED_CHANNELS or ch not in SUPPORTED_CHANNELS:
@@ -340,8 +368,8 @@ def triangle_multiplication(z: torch.Tensor, mask: Optional[torch.Tensor], *, ou
         out = torch.empty_like(z, memory_format=torch.contiguous_format)
     if out.dtype != z.dtype or out.shape != z.shape:
         raise ValueError("out must match z in shape and dtype")
-    ob, _, o_sb = _batch_view(out, "out")
-    m, ms0, ms1, m_sb = _mask_view(mask, z.shape[:-3], n, z.device)
+    _, o_sb, os0, os1 = _pair_strides(out, "out")
+    m, ms0, ms1, m_sb = _mask_args(mask, z, n)
     if z.numel() == 0:
         return out
     f32 = torch.float32
@@ -353,9 +381,9 @@ def triangle_multiplication(z: torch.Tensor, mask: Optional[torch.Tensor], *, ou
         a.compute_dtype = _lib.F32X3
     a.outgoing = 1 if outgoing else 0
     a.add_residual = 1 if add_residual else 0
-    a.z, a.z_s0, a.z_s1 = _ptr(z), zb.stride(1), zb.stride(2)
+    a.z, a.z_s0, a.z_s1 = _ptr(z), zs0, zs1
     a.mask, a.mask_s0, a.mask_s1 = _ptr(m), ms0, ms1
-    a.out, a.out_s0, a.out_s1 = _ptr(out), ob.stride(1), ob.stride(2)
+    a.out, a.out_s0, a.out_s1 = _ptr(out), os0, os1
     a.batch, a.z_sb, a.mask_sb, a.out_sb = nbatch, z_sb, m_sb, o_sb
     keep = [prepared(norm_in_weight, f32), prepared(norm_in_bias, f32),
             prepared(norm_out_weight, f32), prepared(norm_out_bias, f32),

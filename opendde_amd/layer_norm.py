@@ -94,6 +94,13 @@ def _reset_loader_for_tests() -> None:
         _fast_layer_norm_load_error = None
 
 
+def _like(p: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
+    """The bias as the backward entry points take it: they return its gradient
+    in its shape and type and never read its values, so a bias of another
+    type is not converted."""
+    return p if p.dtype == dtype else torch.empty_like(p, dtype=dtype)
+
+
 class FusedLayerNormAffineFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx: Any, input: torch.Tensor, weight: Optional[torch.Tensor],
@@ -133,13 +140,13 @@ class FusedLayerNormAffineFunction(torch.autograd.Function):
                     g, mean, invvar, input_, shape, eps)
             else:
                 grad_input, grad_weight, grad_bias = ext.backward_with_bias_affine(
-                    g, mean, invvar, input_, shape, bias_.to(dtype=d), eps)
+                    g, mean, invvar, input_, shape, _like(bias_, d), eps)
         elif bias_ is None:
             grad_input, grad_weight, grad_bias = ext.backward_with_weight_affine(
                 g, mean, invvar, input_, shape, weight_.to(dtype=d), eps)
         else:
             grad_input, grad_weight, grad_bias = ext.backward_with_both_affine(
-                g, mean, invvar, input_, shape, weight_.to(dtype=d), bias_.to(dtype=d), eps)
+                g, mean, invvar, input_, shape, weight_.to(dtype=d), _like(bias_, d), eps)
         return (grad_input,
                 None if weight_ is None else grad_weight,
                 None if bias_ is None else grad_bias,
