@@ -11,7 +11,7 @@
 // n2 <= 2048): a row is owned by a group of G lanes (G a power of two <= 64)
 // holding NV 16-byte vectors each, so a whole row sits in registers and the
 // two-pass statistics (mean, then sum of squared deviations) read HBM once.
-// The group reduction is an xor butterfly, so every lane of a group ends with
+// The group reduction is a butterfly, so every lane of a group ends with
 // the same bits.  Each group keeps R rows in flight per iteration.  gamma and
 // beta are converted to f32 once per lane and kept in registers.
 //
@@ -85,17 +85,35 @@ __device__ __forceinline__ u32x4 pack(const float* f, f16*) {
   return __builtin_bit_cast(u32x4, h);
 }
 
-template <typename T> __device__ __forceinline__ void load_vec(const T* p, float* f) {
-  unpack(*reinterpret_cast<const u32x4*>(p), f, (T*)nullptr);
+// kNt: the streaming cache policy
+template <bool kNt, typename T>
+__device__ __forceinline__ void load_vec(const T* p, float* f) {
+  const u32x4* q = reinterpret_cast<const u32x4*>(p);
+  unpack(kNt ? load_stream(q) : *q, f, (T*)nullptr);
 }
-template <typename T> __device__ __forceinline__ void store_vec(T* p, const float* f) {
-  *reinterpret_cast<u32x4*>(p) = pack(f, (T*)nullptr);
+template <bool kNt, typename T>
+__device__ __forceinline__ void store_vec(T* p, const float* f) {
+  if constexpr (kNt) store_stream(reinterpret_cast<u32x4*>(p), pack(f, (T*)nullptr));
+  else *reinterpret_cast<u32x4*>(p) = pack(f, (T*)nullptr);
 }
 
-// Sum over the G = 1 << lg lanes of an aligned lane group (xor butterfly:
-// every lane of the group ends with the same value).
+// Sum over the G = 1 << lg lanes of an aligned lane group (every lane of the
+// group ends with the same value): the xor butterfly, its steps of 1 and 2 as
+// quad permutes, of 4 and 8 as mirrors (the lanes of a finished 4 or 8 hold one
+// value, so the mirror's partner serves as well), of 16 and 32 as lane swaps.
+// All are register moves; __shfl_xor goes through the LDS unit.
+template <int kCtrl>
+__device__ __forceinline__ float dpp_add(float s) {
+  return s + __int_as_float(
+                 __builtin_amdgcn_mov_dpp(__float_as_int(s), kCtrl, 0xF, 0xF, true));
+}
 __device__ __forceinline__ float group_sum(float s, int lg) {
-  for (int o = 1; o < (1 << lg); o <<= 1) s += __shfl_xor(s, o);
+  if (lg > 0) s = dpp_add<0xB1>(s);   // quad_perm [1, 0, 3, 2]
+  if (lg > 1) s = dpp_add<0x4E>(s);   // quad_perm [2, 3, 0, 1]
+  if (lg > 2) s = dpp_add<0x141>(s);  // row_half_mirror
+  if (lg > 3) s = dpp_add<0x140>(s);  // row_mirror
+  if (lg > 4) s = swap16_add(s);
+  if (lg > 5) s = swap32_add(s);
   return s;
 }
 
@@ -113,7 +131,7 @@ __device__ __forceinline__ void load_param(const T* p, int j, int lg, int V, flo
   for (int k = 0; k < NV; ++k) {
     const int v = j + (k << lg);
     if (p && v < V) {
-      load_vec(p + v * VEC, f[k]);
+      load_vec<false>(p + v * VEC, f[k]);
     } else {
 #pragma unroll
       for (int e = 0; e < VEC; ++e) f[k][e] = dflt;
@@ -146,7 +164,7 @@ __global__ __launch_bounds__(kLnThreads) void ln_fwd_rows_kernel(
       for (int k = 0; k < NV; ++k) {
         const int v = j + (k << lg);
         if (r < n1 && v < V) {
-          load_vec(x + r * n2 + v * VEC, f[t][k]);
+          load_vec<false>(x + r * n2 + v * VEC, f[t][k]);
         } else {
 #pragma unroll
           for (int e = 0; e < VEC; ++e) f[t][k][e] = 0.0f;
@@ -183,7 +201,7 @@ __global__ __launch_bounds__(kLnThreads) void ln_fwd_rows_kernel(
           float o[VEC];
 #pragma unroll
           for (int e = 0; e < VEC; ++e) o[e] = (f[t][k][e] - mu) * iv * g[k][e] + b[k][e];
-          store_vec(out + r * n2 + v * VEC, o);
+          store_vec<false>(out + r * n2 + v * VEC, o);
         }
       }
       if (j == 0) {
@@ -196,7 +214,7 @@ __global__ __launch_bounds__(kLnThreads) void ln_fwd_rows_kernel(
 
 // grad_input for the rows of each group; optional per-workgroup partial sums
 // part[blockIdx.x][0][c] = sum dout*xhat, part[blockIdx.x][1][c] = sum dout.
-template <typename T, int NV, int R>
+template <typename T, int NV, int R, bool kNt>
 __global__ __launch_bounds__(kLnThreads) void ln_bwd_rows_kernel(
     const T* __restrict__ dout, const T* __restrict__ x, const float* __restrict__ mean,
     const float* __restrict__ invvar, const T* __restrict__ gamma, T* __restrict__ dx,
@@ -231,8 +249,8 @@ __global__ __launch_bounds__(kLnThreads) void ln_bwd_rows_kernel(
       for (int k = 0; k < NV; ++k) {
         const int v = j + (k << lg);
         if (r < n1 && v < V) {
-          load_vec(x + r * n2 + v * VEC, xf[t][k]);
-          load_vec(dout + r * n2 + v * VEC, df[t][k]);
+          load_vec<kNt>(x + r * n2 + v * VEC, xf[t][k]);
+          load_vec<kNt>(dout + r * n2 + v * VEC, df[t][k]);
         } else {
 #pragma unroll
           for (int e = 0; e < VEC; ++e) xf[t][k][e] = df[t][k][e] = 0.0f;
@@ -266,7 +284,7 @@ __global__ __launch_bounds__(kLnThreads) void ln_bwd_rows_kernel(
 #pragma unroll
           for (int e = 0; e < VEC; ++e)
             o[e] = iv[t] * (df[t][k][e] * g[k][e] - s1 - xf[t][k][e] * s2);
-          store_vec(dx + r * n2 + v * VEC, o);
+          store_vec<kNt>(dx + r * n2 + v * VEC, o);
         }
       }
     }
@@ -417,8 +435,19 @@ __global__ __launch_bounds__(1024) void ln_param_grad_reduce_kernel(
   if (!dst) return;  // uniform over the workgroup
   const int c = blockIdx.x * 64 + threadIdx.x;
   float s = 0.0f;
-  if (c < n2)
-    for (int p = threadIdx.y; p < nparts; p += 16) s += part[(int64_t(p) * 2 + blockIdx.y) * n2 + c];
+  if (c < n2) {
+    // eight loads in flight, added in order
+    const float* src = part + int64_t(blockIdx.y) * n2 + c;
+    int p = threadIdx.y;
+    for (; p + 7 * 16 < nparts; p += 8 * 16) {
+      float v[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v[k] = src[int64_t(p + 16 * k) * 2 * n2];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) s += v[k];
+    }
+    for (; p < nparts; p += 16) s += src[int64_t(p) * 2 * n2];
+  }
   acc[threadIdx.y][threadIdx.x] = s;
   __syncthreads();
   for (int h = 8; h > 0; h >>= 1) {
@@ -431,6 +460,16 @@ __global__ __launch_bounds__(1024) void ln_param_grad_reduce_kernel(
 // ---------------------------------------------------------------------------
 // host planning
 // ---------------------------------------------------------------------------
+
+// Rows a lane group loads at once: two where a row is one vector a lane.  The
+// forward runs four workgroups per CU there (eight for wider rows), the
+// backward four: fewer streams read at a time keep more DRAM pages open.  us,
+// 1048576 x 128, bf16 forward at 1 / 2 / 4 / 8 rows: 99 / 103 / 103 / 106 with
+// four workgroups per CU, 102 / 102 / 120 / 111 with eight (f32, four: 245 /
+// 186 / 228 / 246); bf16 backward 168 / 155 / 156 with four, 178 / 162 / 163
+// with eight.  Two vectors a lane, 131072 x 1000: 1 / 2 rows forward 93 / 94,
+// backward 155 / 235.
+constexpr int ln_rows_in_flight(int nv) { return nv == 1 ? 2 : 1; }
 
 struct LnPlan {
   bool rows = false;  // row kernels (else generic)
@@ -473,9 +512,9 @@ LnPlan plan_shape(int64_t n1, int n2, int dt, bool backward) {
     p.rows = p.nv > 0;
   }
   if (p.rows) {
-    p.r = p.nv == 1 ? 4 : p.nv == 2 ? 2 : 1;
+    p.r = ln_rows_in_flight(p.nv);
     const int64_t rows_per_block = int64_t(kLnThreads >> p.lg) * p.r;
-    const int64_t cap = backward ? kLnBwdMaxBlocks : kLnFwdMaxBlocks;
+    const int64_t cap = backward ? kLnBwdMaxBlocks : p.nv <= 2 ? kLnFwdMaxBlocks / 2 : kLnFwdMaxBlocks;
     p.blocks = std::min<int64_t>((n1 + rows_per_block - 1) / rows_per_block, cap);
     p.nparts = p.blocks;
   } else {
@@ -485,11 +524,18 @@ LnPlan plan_shape(int64_t n1, int n2, int dt, bool backward) {
   return p;
 }
 
+// The backward reads two tensors and writes one: past half the 256 MB of the
+// last-level cache a tensor, the streaming policy is the faster (268 MB tensors
+// 159 us against 171, 134 MB 91 / 93; 67 MB 52 / 48), by more than the next
+// forward loses that finds less of its input in that cache (349525 x 384 bf16:
+// 23 against 4 us).  The forward gains nothing from it.
+inline bool ln_streams(int64_t n1, int n2, int es) { return n1 * n2 * es >= int64_t(128) << 20; }
+
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 template <typename T, int NV>
 void launch_fwd_rows(const LnPlan& p, const odde_layer_norm_args* a, hipStream_t st) {
-  constexpr int R = NV == 1 ? 4 : NV == 2 ? 2 : 1;
+  constexpr int R = ln_rows_in_flight(NV);
   hipLaunchKernelGGL((ln_fwd_rows_kernel<T, NV, R>), dim3(p.blocks), dim3(kLnThreads), 0, st,
                      (const T*)a->x, (const T*)a->gamma, (const T*)a->beta, (T*)a->out, a->mean,
                      a->invvar, a->n1, a->n2, p.lg, a->eps);
@@ -498,10 +544,12 @@ void launch_fwd_rows(const LnPlan& p, const odde_layer_norm_args* a, hipStream_t
 template <typename T, int NV>
 void launch_bwd_rows(const LnPlan& p, const odde_layer_norm_bwd_args* a, float* part,
                      hipStream_t st) {
-  constexpr int R = NV == 1 ? 4 : NV == 2 ? 2 : 1;
-  hipLaunchKernelGGL((ln_bwd_rows_kernel<T, NV, R>), dim3(p.blocks), dim3(kLnThreads), 0, st,
-                     (const T*)a->dout, (const T*)a->x, a->mean, a->invvar, (const T*)a->gamma,
-                     (T*)a->grad_input, part, a->n1, a->n2, p.lg);
+  constexpr int R = ln_rows_in_flight(NV);
+  const auto kernel = ln_streams(a->n1, a->n2, sizeof(T)) ? ln_bwd_rows_kernel<T, NV, R, true>
+                                                          : ln_bwd_rows_kernel<T, NV, R, false>;
+  hipLaunchKernelGGL(kernel, dim3(p.blocks), dim3(kLnThreads), 0, st, (const T*)a->dout,
+                     (const T*)a->x, a->mean, a->invvar, (const T*)a->gamma, (T*)a->grad_input,
+                     part, a->n1, a->n2, p.lg);
 }
 
 template <typename T>
