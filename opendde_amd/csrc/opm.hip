@@ -47,9 +47,9 @@ struct OpmTile {
 // 256 x 256 GEMM tiles staged 64 MSA rows at a time (whole 128-byte lines),
 // one workgroup per CU; the 64 pairs' blocks reuse the stage buffers.
 using OpmTileBig = OpmTile<8, 8, 2, 2, 64>;
-// 256 x 128 GEMM tiles staged 32 MSA rows at a time, two workgroups per CU.
-using OpmTileSmall = OpmTile<8, 4, 4, 3, 32>;
-using OpmTileUsed = OpmTileBig;  // measured 3.20 vs 3.69 ms at S=1280, N=1024
+// (256 x 128 tiles staged 32 rows at a time, two workgroups per CU: 3.69 ms
+// against 3.20 at S=1280, N=1024)
+using OpmTileUsed = OpmTileBig;
 
 struct OpmProjArgs {
   const void* m;
@@ -116,30 +116,31 @@ __global__ __launch_bounds__(256) void opm_proj_kernel(OpmProjArgs a) {
   }
 }
 
-// norm[i][j] = sum_s maskT[i][s] maskT[j][s] + eps over 128 x 128 tiles
-// (grid (Np / 128)^2, 512 threads).
-__global__ __launch_bounds__(512) void opm_norm_kernel(const bf16* __restrict__ maskt, int Np, int Sp,
-                                                       float eps, float* __restrict__ norm) {
-  using S = GemmShape<128, 128, 2>;
+// norm[i][j] = sum_s maskT[i][s] maskT[j][s] + eps over 64 x 64 tiles (grid
+// nt^2, 512 threads).  A chain of Sp / 64 short stages, bound by their latency:
+// at N = 384, S = 1280 36 workgroups of 20 stages, where 128 x 128 tiles of 32
+// rows a stage were 9 of 40 (17 us).
+__global__ __launch_bounds__(512) void opm_norm_kernel(const bf16* __restrict__ maskt, int nt,
+                                                       int Np, int Sp, float eps,
+                                                       float* __restrict__ norm) {
+  using S = GemmShape<64, 64, 2, 64>;
   __shared__ __attribute__((aligned(16))) bf16 sm[3 * S::STAGE_ELEMS];
-  const int nt = Np / 128, ti = blockIdx.x / nt, tj = blockIdx.x % nt;
-  const bf16* A = maskt + (size_t)ti * 128 * Sp;
-  const bf16* B = maskt + (size_t)tj * 128 * Sp;
+  const int ti = blockIdx.x / nt, tj = blockIdx.x % nt;
+  const bf16* A = maskt + (size_t)ti * 64 * Sp;
+  const bf16* B = maskt + (size_t)tj * 64 * Sp;
   f32x4 acc[S::MX][S::MY];
-  gemm_nt_mainloop<128, 128, 2, 3, true>([&](int r) { return A + (size_t)r * Sp; },
-                                         [&](int r) { return B + (size_t)r * Sp; }, Sp, sm, acc);
-  // acc[mi][mj]: column (lane % 16) = row i, values = 4 consecutive j
+  gemm_nt_mainloop<64, 64, 2, 3, true, 64>([&](int r) { return A + (size_t)r * Sp; },
+                                           [&](int r) { return B + (size_t)r * Sp; }, Sp, sm, acc);
+  // acc[mi][0]: column (lane % 16) = row i, values = 4 consecutive j
   const int w = wave_id(), l = lane_id(), g = l >> 4, r16 = l & 15;
   const int wx = w % 2, wy = w / 2;
 #pragma unroll
-  for (int mi = 0; mi < S::MX; ++mi)
-#pragma unroll
-    for (int mj = 0; mj < S::MY; ++mj) {
-      const int i = ti * 128 + wx * 64 + 16 * mi + r16;
-      const int j = tj * 128 + wy * 32 + 16 * mj + 4 * g;
-      store4(norm + (size_t)i * Np + j, acc[mi][mj][0] + eps, acc[mi][mj][1] + eps,
-             acc[mi][mj][2] + eps, acc[mi][mj][3] + eps);
-    }
+  for (int mi = 0; mi < S::MX; ++mi) {
+    const int i = ti * 64 + wx * 32 + 16 * mi + r16;
+    const int j = tj * 64 + wy * 16 + 4 * g;
+    store4(norm + (size_t)i * Np + j, acc[mi][0][0] + eps, acc[mi][0][1] + eps,
+           acc[mi][0][2] + eps, acc[mi][0][3] + eps);
+  }
 }
 
 struct OpmOuterArgs {
@@ -150,6 +151,7 @@ struct OpmOuterArgs {
   const float* b_out;  // [c_z] or null
   void* out;           // [N][N][c_z]
   int S, N, Np, Sp, add;
+  int nt;              // tile rows and columns of the grid
   float eps;
 };
 
@@ -184,13 +186,25 @@ __global__ __launch_bounds__(512) void opm_outer_kernel(OpmOuterArgs a) {
   __shared__ __attribute__((aligned(16))) bf16 sm[TL::LDS_BYTES / 2];
   const int w = wave_id(), l = lane_id(), g = l >> 4, r16 = l & 15;
   int ti, tj;
-  opm_tile_map(blockIdx.x, a.Np / TI, a.Np / TJ, ti, tj);
+  opm_tile_map(blockIdx.x, a.nt, a.nt, ti, tj);
+  if (ti * TI >= a.N || tj * TJ >= a.N) return;  // rounding of the bands
   const bf16* A = a.at + (size_t)ti * TI * kOpmC * a.Sp;
   const bf16* B = a.bt + (size_t)tj * TJ * kOpmC * a.Sp;
   f32x4 acc[S::MX][S::MY];
-  gemm_nt_mainloop<TI * kOpmC, TJ * kOpmC, TL::WX, TL::NS, true, TL::KC>(
-      [&](int r) { return A + (size_t)r * a.Sp; }, [&](int r) { return B + (size_t)r * a.Sp; },
-      a.Sp, sm, acc);
+  auto arow = [&](int r) { return A + (size_t)r * a.Sp; };
+  auto brow = [&](int r) { return B + (size_t)r * a.Sp; };
+  if (a.Sp > 0 && a.Sp <= (1 << 22)) {  // 32-bit offsets within a tile's rows
+    GemmBufs bufs;
+    bufs.a = A;
+    bufs.a_bytes = (uint32_t)((size_t)TI * kOpmC * a.Sp * sizeof(bf16));
+    bufs.b = B;
+    bufs.b_bytes = (uint32_t)((size_t)TJ * kOpmC * a.Sp * sizeof(bf16));
+    gemm_nt_mainloop_pipe64_k<TI * kOpmC, TJ * kOpmC, TL::WX, true, true>(
+        arow, brow, a.Sp / 64, [](bool, int st) { return st * 64; }, sm, acc, bufs);
+  } else {
+    gemm_nt_mainloop<TI * kOpmC, TJ * kOpmC, TL::WX, TL::NS, true, TL::KC>(arow, brow, a.Sp, sm,
+                                                                           acc);
+  }
   // acc[mi][mj]: column (lane % 16) = A row 32 RI wx + 16 mi + r16 (residue
   // RI wx + mi / 2, c1 = 16 (mi % 2) + r16); values e = B rows
   // 32 RJ wy + 16 mj + 4 g + e (residue RJ wy + mj / 2, c2 = 16 (mj % 2) + 4 g + e)
@@ -294,7 +308,7 @@ int run_opm(const odde_opm_args* a, hipStream_t st) {
     p.w12 = static_cast<const bf16*>(a->w_12);
     p.at = at; p.bt = bt; p.maskt = maskt;
     p.S = S; p.N = N; p.Sp = Sp; p.eps = a->ln_eps;
-    dim3 grid(Sp / kOpmSB, Np);
+    dim3 grid(Sp / kOpmSB, round_up(N, OpmTileUsed::TI));
     switch (a->c_m) {
       case 32: hipLaunchKernelGGL((opm_proj_kernel<MT, 32>), grid, dim3(256), 0, st, p); break;
       case 64: hipLaunchKernelGGL((opm_proj_kernel<MT, 64>), grid, dim3(256), 0, st, p); break;
@@ -305,8 +319,8 @@ int run_opm(const odde_opm_args* a, hipStream_t st) {
     if (rc) return rc;
   }
   if (norm) {
-    const int nt = Np / 128;
-    hipLaunchKernelGGL(opm_norm_kernel, dim3(nt * nt), dim3(512), 0, st, maskt, Np, Sp, a->eps,
+    const int nt = (N + 63) / 64;
+    hipLaunchKernelGGL(opm_norm_kernel, dim3(nt * nt), dim3(512), 0, st, maskt, nt, Np, Sp, a->eps,
                        norm);
     int rc = check_launch("opm_norm");
     if (rc) return rc;
@@ -318,7 +332,13 @@ int run_opm(const odde_opm_args* a, hipStream_t st) {
   q.out = a->out;
   q.S = S; q.N = N; q.Np = Np; q.Sp = Sp; q.add = a->add_residual; q.eps = a->eps;
   using TL = OpmTileUsed;
-  const unsigned tiles = (unsigned)(Np / TL::TI) * (unsigned)(Np / TL::TJ);
+  static_assert(TL::TI == TL::TJ, "square tiles");
+  // Only tiles that hold residues (the buffers are laid out for N rounded up to
+  // 128: at N = 151 that is 2.8 times as many), rounded up to whole bands of 8
+  // where that lets every XCD take its own (opm_tile_map).
+  const int nt = (N + TL::TI - 1) / TL::TI, nt8 = round_up(nt, 8);
+  q.nt = (nt8 / 8) * (nt8 / 8) % 8 == 0 ? nt8 : nt;
+  const unsigned tiles = (unsigned)q.nt * (unsigned)q.nt;
   switch (a->c_z) {
     case 64: hipLaunchKernelGGL((opm_outer_kernel<OT, 64, TL>), dim3(tiles), dim3(512), 0, st, q); break;
     case 128: hipLaunchKernelGGL((opm_outer_kernel<OT, 128, TL>), dim3(tiles), dim3(512), 0, st, q); break;

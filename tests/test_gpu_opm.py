@@ -76,6 +76,24 @@ def test_outer_product_mean_matches_oracle(S, N, c_m, c_z, masked):
     assert_bf16(got.float(), exp, f"opm S={S} N={N} c_m={c_m} c_z={c_z}")
 
 
+@pytest.mark.parametrize("S,N,masked", [(3, 1, True), (70, 9, True), (129, 66, True),
+                                        (64, 201, True), (65, 201, False)])
+def test_outer_product_mean_tiles(S, N, masked):
+    """Only tiles that hold residues run (N of 8 and 64 and one more; bands
+    rounded past the last tile at N = 201), over a workspace of NaN: the rows of
+    the padded layout that nothing writes must not reach the result."""
+    say(f"[gpu] opm tiles S={S} N={N} mask={masked}")
+    mod = _module(64, 128, 77 + S + N)
+    m, mask = _inputs(S, N, 64, S + N, masked)
+    exp = ref.outer_product_mean(m.float(), mask, params_of(mod))
+    mod, m, mask = mod.to(DEV), m.to(DEV), None if mask is None else mask.to(DEV)
+    torch.cuda.empty_cache()
+    dirty = torch.full((1 << 26,), float("nan"), device=DEV)
+    del dirty  # its block serves the call's workspace
+    got = mod(m, mask, kernel="hip")
+    assert_bf16(got, exp, f"opm tiles S={S} N={N} mask={masked}")
+
+
 def test_outer_product_mean_fp32_msa_under_autocast_and_residual_add():
     """fp32 MSA under bf16 autocast, and the MSA module's z += update fused
     into the kernel for an fp32 and a bf16 pair tensor."""
