@@ -118,15 +118,17 @@ __device__ __forceinline__ void astat_rows_ready(Frag<bf16> (&A)[MB][KT]) {
 //   kPairCols = true : column (lane % 16) is the row, its 4 values are weight
 //                      rows 16 j + 4 (lane / 16) + e;
 //   kPairCols = false: the transpose.
-template <int MB, int KT, bool kPairCols>
-__device__ __forceinline__ void astat_mult(const bf16* buf, int l, const Frag<bf16> (&A)[MB][KT],
-                                           f32x4 (&acc)[MB][2]) {
+// A0 meets the first 16 weight rows, A1 the others.
+// AH weight fragments are read ahead.
+template <int MB, int KT, bool kPairCols, int AH = 8 / MB>
+__device__ __forceinline__ void astat_mult(const bf16* buf, int l, const Frag<bf16> (&A0)[MB][KT],
+                                           const Frag<bf16> (&A1)[MB][KT], f32x4 (&acc)[MB][2]) {
   const int g = l >> 4, r16 = l & 15;
   const bf16* p0 = buf + r16 * 64 + ((g ^ (r16 & 7)) * 8);        // even k steps
   const bf16* p1 = buf + r16 * 64 + (((4 + g) ^ (r16 & 7)) * 8);  // odd ones
   // fragment u = (k step u / 2, weight block u % 2): the one read while u is
-  // multiplied is 8 MFMAs ahead (u + 2 at MB = 4)
-  constexpr int AH = 8 / MB, NB = AH + 1;
+  // multiplied is u + AH, by default 8 MFMAs ahead
+  constexpr int NB = AH + 1;
   Frag<bf16> b[NB];
   auto read = [&](int u) {
     const int t = u >> 1;
@@ -143,8 +145,9 @@ __device__ __forceinline__ void astat_mult(const bf16* buf, int l, const Frag<bf
     if (u + AH < 2 * KT) read(u + AH);
 #pragma unroll
     for (int i = 0; i < MB; ++i) {
-      if constexpr (kPairCols) mma(acc[i][u & 1], b[u % NB], A[i][u >> 1]);
-      else mma(acc[i][u & 1], A[i][u >> 1], b[u % NB]);
+      const Frag<bf16>& row = (u & 1) ? A1[i][u >> 1] : A0[i][u >> 1];
+      if constexpr (kPairCols) mma(acc[i][u & 1], b[u % NB], row);
+      else mma(acc[i][u & 1], row, b[u % NB]);
     }
   }
   __builtin_amdgcn_sched_group_barrier(0x100, AH, 0);
@@ -153,7 +156,13 @@ __device__ __forceinline__ void astat_mult(const bf16* buf, int l, const Frag<bf
     __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
     __builtin_amdgcn_sched_group_barrier(0x008, MB, 0);
   }
-  __builtin_amdgcn_sched_group_barrier(0x008, 8, 0);
+  __builtin_amdgcn_sched_group_barrier(0x008, AH * MB, 0);
+}
+
+template <int MB, int KT, bool kPairCols>
+__device__ __forceinline__ void astat_mult(const bf16* buf, int l, const Frag<bf16> (&A)[MB][KT],
+                                           f32x4 (&acc)[MB][2]) {
+  astat_mult<MB, KT, kPairCols>(buf, l, A, A, acc);
 }
 
 // Stages 0 .. nst - 1.  wsrc(st): uniform pointer to the first of the weight
@@ -162,18 +171,20 @@ __device__ __forceinline__ void astat_mult(const bf16* buf, int l, const Frag<bf
 // stage(st, buf) multiplies and stores; it is called by live waves only and
 // issues kStores vector stores or more, after which the next stage's loads
 // are the only older ones it has to wait for.  sm holds two stage buffers;
-// l: astat_lane().
+// l: astat_lane().  kStores < 0: any number of them, on three stage buffers:
+// the loads run two stages ahead, and a stage waits until no more operations
+// are out than the next stage's loads.
 template <int KT, int kStores, typename WSrc, typename RowOf, typename Stage>
 __device__ __forceinline__ void astat_loop(int nst, bool live, bf16* sm, int l, WSrc wsrc, RowOf row_of,
                                            Stage stage) {
   using S = AstatShape<4, KT>;  // the stages do not depend on MB
-  constexpr int C = KT * 32;
+  constexpr int C = KT * 32, NB = kStores < 0 ? 3 : 2;
   const int lr = l >> 3;
   const int w = __builtin_amdgcn_readfirstlane(wave_id());
   const uint32_t voff = (uint32_t)(row_of(lr) * C + (((l & 7) ^ lr) * 8)) * (uint32_t)sizeof(bf16);
   auto issue = [&](int st) {
     const bf16* src = wsrc(st);
-    bf16* dst = sm + (st & 1) * S::STAGE + w * 512;
+    bf16* dst = sm + (st % NB) * S::STAGE + w * 512;
 #pragma unroll
     for (int k = 0; k < S::LOADS; ++k)
       buffer_load_lds16(src, 12 * C * (uint32_t)sizeof(bf16), dst + k * (kAsCols * 64), voff,
@@ -182,10 +193,23 @@ __device__ __forceinline__ void astat_loop(int nst, bool live, bf16* sm, int l, 
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   barrier_nofence();  // the buffers are free (an earlier loop's last stage)
   issue(0);
+  if constexpr (kStores < 0) {
+    if (nst > 1) issue(1);
+    for (int st = 0; st < nst; ++st) {
+      if (st + 1 < nst) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(S::LOADS) : "memory");
+      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // own reads of stage st - 1 done
+      barrier_nofence();
+      if (st + 2 < nst) issue(st + 2);  // the buffer last read in stage st - 1
+      __builtin_amdgcn_sched_barrier(0);
+      if (live) stage(st, sm + (st % NB) * S::STAGE);
+    }
+    return;
+  }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   for (int st = 0; st < nst; ++st) {
     if (st) {  // this wave's loads of stage st landed; its last stores may not have
-      if (live) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kStores) : "memory");
+      if (live) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kStores < 0 ? 0 : kStores) : "memory");
       else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // own reads of stage st - 1 done

@@ -1232,6 +1232,87 @@ __global__ __launch_bounds__(512) void trimul_out_wide_kernel(TrimulWideOutArgs<
   }
 }
 
+// The same for C = Ch = 32 KT, row-stationary (astat.hpp): a wave holds its 32
+// rows of both operands, a stage is 16 rows of W_z (LDS rows 0-15) and the same
+// 16 of W_g.  A row's fp32 results of two stages are its 128-byte line, stored
+// whole.  LDS bound: a weight fragment serves 32 rows, an LDS cycle for every
+// MFMA cycle, but each operand is read once for all channels and two workgroups
+// share a CU.  C = 384, N = 517: 337 -> 285 us against 256 x 128 tiles (two
+// mainloops of K = 384), 615 TF/s.  gridDim: row tiles of 128 x csplit.
+template <int KT, typename ZT>
+__global__ __launch_bounds__(256, 2) void trimul_out_rows_kernel(TrimulWideOutArgs<ZT> a,
+                                                                 int csplit) {
+  constexpr int C = KT * 32;
+  constexpr bool kLines = std::is_same<ZT, float>::value;
+  __shared__ __attribute__((aligned(16))) bf16 sm[3 * AstatShape<2, KT>::STAGE];
+  int rt, ct;
+  wide_tile_map(blockIdx.x, csplit, rt, ct);
+  const int np = a.np, n = a.n;
+  const int64_t x0 = (int64_t)rt * 128;
+  if (x0 >= (int64_t)n * np) return;
+  const int w = __builtin_amdgcn_readfirstlane(wave_id());
+  const int l = astat_lane(), g = l >> 4, r16 = l & 15;
+  const int64_t mw = x0 + 32 * w;  // the wave's 32 pairs lie in one row x
+  const int x = (int)(mw / np), yw = (int)(mw % np);
+  const bool live = x < n && yw < n;
+  Frag<bf16> P[2][KT], Z[2][KT];
+  astat_load_rows<2, KT>([&](int i) { return a.pn + (mw + 16 * i + r16) * C; }, l, P);
+  astat_load_rows<2, KT>(
+      [&](int i) {
+        const int y = yw + 16 * i + r16;  // the incoming form's z rows were normalised transposed
+        const int64_t zr = !a.zn_transposed ? mw + 16 * i + r16
+                           : x < n && y < n ? (int64_t)y * np + x
+                                            : 0;
+        return a.zn + zr * C;
+      },
+      l, Z);
+  astat_rows_ready<2, KT>(P);
+  astat_rows_ready<2, KT>(Z);
+  const int nst = C / 16 / csplit, st0 = ct * nst;  // nst is even
+  const bf16* W = ((w & 2) ? a.wg : a.wz) + (size_t)(st0 * 16 + 8 * (w & 1)) * C;
+  // rows y and y ^ 1 (lanes r16, r16 ^ 1) complete each other's lines
+  const ZT* zx = a.z + (int64_t)x * a.z_s0 + (int64_t)yw * a.z_s1 + st0 * 16;
+  ZT* ox = a.out + (int64_t)x * a.o_s0 + (int64_t)yw * a.o_s1 + st0 * 16;
+  float held[2][4];
+  astat_loop<KT, -1>(
+      nst, live, sm, l, [&](int st) { return W + (size_t)st * 16 * C; }, [](int r) { return r; },
+      [&](int st, const bf16* buf) __attribute__((always_inline)) {
+        // lane pointers formed anew: kept across the stage they would not fit
+        const int sl = astat_lane(), sg = sl >> 4, sr = sl & 15;
+        const ZT* zl = zx + (int64_t)sr * a.z_s1 + 4 * sg;
+        ZT* ol = ox + (int64_t)sr * a.o_s1;
+        float r[2][4];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          r[i][0] = r[i][1] = r[i][2] = r[i][3] = 0.f;
+          if (a.add && yw + 16 * i + sr < n)
+            load4(zl + (int64_t)(16 * i) * a.z_s1 + 16 * st, r[i]);
+        }
+        f32x4 acc[2][2];
+        astat_mult<2, KT, true, 3>(buf, l, P, Z, acc);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const int y = yw + 16 * i + sr;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) r[i][e] += sigmoidf_(acc[i][1][e]) * acc[i][0][e];
+          ZT* own = ol + (int64_t)(16 * i) * a.o_s1;
+          if constexpr (!kLines) {
+            if (y < n) store4(own + 16 * st + 4 * sg, r[i][0], r[i][1], r[i][2], r[i][3]);
+          } else if (st & 1) {
+            const int c0 = 16 * (st - 1);
+            ZT* partner = own + ((sr & 1) ? -a.o_s1 : a.o_s1);
+            store_line_pair(reinterpret_cast<f32x4*>(own + c0),
+                            reinterpret_cast<f32x4*>(partner + c0), sg,
+                            f32x4{held[i][0], held[i][1], held[i][2], held[i][3]},
+                            f32x4{r[i][0], r[i][1], r[i][2], r[i][3]}, y < n, (y ^ 1) < n);
+          } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) held[i][e] = r[i][e];
+          }
+        }
+      });
+}
+
 }  // namespace odde
 
 // ===========================================================================
@@ -1374,6 +1455,16 @@ int run_trimul_wide(const odde_trimul_args* a, const TrimulWs& ws, hipStream_t s
     o.out = static_cast<ZT*>(a->out); o.o_s0 = a->out_s0; o.o_s1 = a->out_s1;
     o.n = n; o.np = np; o.c = C; o.ch = ch; o.add = a->add_residual;
     o.zn_transposed = outgoing ? 0 : 1;
+    if (C == ch && C > 128) {
+      const int rt = (int)(rows / 128), csplit = astat_csplit(rt, C / 32, 256);
+      if (C == 256)
+        hipLaunchKernelGGL((trimul_out_rows_kernel<8, ZT>), dim3(rt * csplit), dim3(256), 0, st, o,
+                           csplit);
+      else
+        hipLaunchKernelGGL((trimul_out_rows_kernel<12, ZT>), dim3(rt * csplit), dim3(256), 0, st,
+                           o, csplit);
+      return check_launch("trimul_out (rows)");
+    }
     const int ncol = C / kWTY;
     hipLaunchKernelGGL((trimul_out_wide_kernel<ZT>), dim3(row_tiles * ncol), dim3(512), 0, st, o,
                        ncol);
