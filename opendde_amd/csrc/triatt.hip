@@ -2064,11 +2064,18 @@ void launch_proj(const TriattProjArgs<ZT, CT>& p, int n, int jp, hipStream_t st)
   // large enough (n >= 256)
   constexpr int kRB = sizeof(CT) != 4 ? 1 : kC <= 8 ? 2 : 1;
   if constexpr (sizeof(CT) == 4 && kC <= 4) {
-    // f32 data from n = 256: the weights staged in LDS
-    if (n >= 256 && !triatt_proj_f32_plain()) {
-      dim3 grid(jp / 64, (n + 1) / 2);
-      hipLaunchKernelGGL((triatt_proj_kernel<ZT, CT, kC, 2, kX3Mul, true>), grid, dim3(256), 0, st,
-                         p);
+    // f32 data from n = 112: the weights staged in LDS, two rows i per
+    // workgroup from n = 193.  C = 128, us, by fragment with channel splits /
+    // staged one row / two, fp32: n = 90 41 / 47 / 66, 128 53 / 46 / 66, 160 87 /
+    // 66 / 69, 200 145 / 113 / 104, 250 152 / 117 / 104; three parts: 128 50 /
+    // 37 / 43, 160 84 / 44 / 45, 200 140 / 68 / 56.
+    if (n >= 112 && !triatt_proj_f32_plain()) {
+      if (n <= 192)
+        hipLaunchKernelGGL((triatt_proj_kernel<ZT, CT, kC, 1, kX3Mul, true>), dim3(jp / 64, n),
+                           dim3(256), 0, st, p);
+      else
+        hipLaunchKernelGGL((triatt_proj_kernel<ZT, CT, kC, 2, kX3Mul, true>),
+                           dim3(jp / 64, (n + 1) / 2), dim3(256), 0, st, p);
       return;
     }
   }
@@ -2159,23 +2166,39 @@ inline bool triatt_out_f32_plain() {
 }
 template <typename ZT, typename CT, int kHD>
 void launch_out(const TriattOutArgs<ZT, CT>& p, int n, int jp, bool x3, hipStream_t st) {
-  // fp32: W_o is read from L2 per fragment, so 4 rows i per workgroup up to
-  // HD = 128 (2 up to 256) once the grid stays large (n >= 256)
+  if constexpr (sizeof(CT) == 4 && kHD <= 4) {
+    // f32 data from n = 65: W_o staged in LDS, for one row i per workgroup up
+    // to n = 192, two above.  C = HD = 128, us, by fragment with channel splits /
+    // staged one row / two / four, fp32: n = 64 7.9 / 12 / 17 / 29, 90 16 / 13 /
+    // 18 / 29, 160 29 / 19 / 20 / 30, 250 48 / 30 / 29 / 33, 300 - / 40 / 39 / 50, 640
+    // two / four 133 / 166.
+    if (n > 64 && !triatt_out_f32_plain()) {
+      auto launch = [&](auto x3_c, auto rb_c) {
+        constexpr int RB = decltype(rb_c)::value;
+        hipLaunchKernelGGL((triatt_out_kernel<ZT, CT, kHD, decltype(x3_c)::value, RB, true>),
+                           dim3(jp / 64, (n + RB - 1) / RB), dim3(256), 0, st, p);
+      };
+      using R1 = std::integral_constant<int, 1>;
+      using R2 = std::integral_constant<int, 2>;
+      using R4 = std::integral_constant<int, 4>;
+      // four where the rows i are the ones next to each other in memory (the
+      // ending node), and at HD = 64 from n = 400 (509: 35 us against 41)
+      const bool r4 = n >= 256 && (p.o_s0 < p.o_s1 || (kHD == 2 && n >= 400));
+      if (x3 && n <= 192) launch(std::true_type{}, R1{});
+      else if (x3 && !r4) launch(std::true_type{}, R2{});
+      else if (x3) launch(std::true_type{}, R4{});
+      else if (n <= 192) launch(std::false_type{}, R1{});
+      else if (!r4) launch(std::false_type{}, R2{});
+      else launch(std::false_type{}, R4{});
+      return;
+    }
+  }
+  // W_o read from L2 per fragment: 4 rows i per workgroup up to HD = 128 (2 up
+  // to 256) once the grid stays large (n >= 256)
   constexpr int kRB = sizeof(CT) != 4 ? 1 : kHD <= 4 ? 4 : kHD <= 8 ? 2 : 1;
   if constexpr (kRB > 1) {
     if (n >= 256) {
       const int rows = (n + kRB - 1) / kRB;
-      if (kHD <= 4 && !triatt_out_f32_plain()) {
-        // f32 data: W_o staged in LDS (one split)
-        dim3 grid(jp / 64, rows);
-        if (x3)
-          hipLaunchKernelGGL((triatt_out_kernel<ZT, CT, kHD, true, kRB, true>), grid, dim3(256), 0,
-                             st, p);
-        else
-          hipLaunchKernelGGL((triatt_out_kernel<ZT, CT, kHD, false, kRB, true>), grid, dim3(256), 0,
-                             st, p);
-        return;
-      }
       dim3 grid(jp / 64, rows, proj_split((int64_t)(jp / 64) * rows, p.c / 16));
       if (x3)
         hipLaunchKernelGGL((triatt_out_kernel<ZT, CT, kHD, true, kRB>), grid, dim3(256), 0, st, p);

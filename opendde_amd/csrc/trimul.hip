@@ -1519,8 +1519,18 @@ void launch_tp(const TrimulProjArgs<ZT, CT>& p, hipStream_t st) {
   // planes (Np is a multiple of kRB)
   constexpr int kRB = sizeof(CT) != 4 ? 1 : kC <= 4 ? 4 : kC <= 8 ? 2 : 1;
   if constexpr (sizeof(CT) == 4 && kC <= 4) {
-    // f32 data from N = 129: the weights staged in LDS (kSRB row blocks
-    // per wave)
+    // f32 data from N = 65: the weights staged in LDS, for one first index x per
+    // workgroup up to N = 128, kSRB above.  C = 128, us, by fragment with channel
+    // splits / staged one / two, fp32: N = 64 16 / 27 / 44, 90 33 / 30 / 46, 128
+    // 43 / 31 / 47, 160 - / 50 / 49; three parts: 64 16 / 17 / 22, 90 31 / 19 / 23,
+    // 128 44 / 19 / 24.
+    if constexpr (!kX3Out) {  // (the three-part contraction starts at N = 129)
+      if (p.n > 64 && p.n <= 128 && !trimul_proj_f32_plain()) {
+        hipLaunchKernelGGL((trimul_proj_kernel<ZT, CT, kC, 1, false, kX3Mul, true>),
+                           dim3(p.np / 64, p.n), dim3(256), 0, st, p);
+        return;
+      }
+    }
     if (p.n > 128 && !trimul_proj_f32_plain()) {
       dim3 grid(p.np / 64, (p.n + kSRB - 1) / kSRB);
       hipLaunchKernelGGL((trimul_proj_kernel<ZT, CT, kC, kSRB, kX3Out, kX3Mul, true>), grid,
@@ -1614,12 +1624,13 @@ template <typename ZT, typename CT, int kC, int kCh>
 void launch_to(const TrimulOutArgs<ZT, CT>& p, bool x3, hipStream_t st) {
   if constexpr (sizeof(CT) == 4) {
     if (x3) {
-      // three-part products: the weights staged in LDS from N = 256 (C =
-      // Ch = 128 at N = 1024: 1.24 -> 1.17 ms with two first indices per
-      // workgroup sharing each L2 fragment read, which the staged form
-      // replaces)
+      // three-part products: the weights staged in LDS from N = 65 (C = Ch =
+      // 128, us, by fragment / staged: N = 64 15 / 17, 90 33 / 17, 128 37 / 18,
+      // 200 80 / 38, 250 95 / 40; N = 1024: 1.24 -> 1.17 ms with two first
+      // indices per workgroup sharing each L2 fragment read, which the staged
+      // form replaces)
       if constexpr (kC <= 4 && kCh <= 4) {
-        if (p.n >= 256 && !trimul_out_f32_plain()) {
+        if (p.n > 64 && !trimul_out_f32_plain()) {
           hipLaunchKernelGGL((trimul_out_f32s_kernel<ZT, kC, kCh, true>), dim3(p.np / 64, p.n),
                              dim3(256), 0, st, p);
           return;
@@ -1634,9 +1645,10 @@ void launch_to(const TrimulOutArgs<ZT, CT>& p, bool x3, hipStream_t st) {
     }
   }
   if constexpr (sizeof(CT) == 4 && kC <= 4 && kCh <= 4) {
-    // true fp32 products from N = 256: weights staged in LDS (the grid no
-    // longer needs an output-channel split)
-    if (p.n >= 256 && !trimul_out_f32_plain()) {
+    // true fp32 products from N = 65: weights staged in LDS (us, by fragment
+    // with an output-channel split / staged: N = 64 15 / 21, 90 34 / 22, 128 37 /
+    // 23, 200 81 / 59, 250 91 / 61)
+    if (p.n > 64 && !trimul_out_f32_plain()) {
       hipLaunchKernelGGL((trimul_out_f32s_kernel<ZT, kC, kCh>), dim3(p.np / 64, p.n), dim3(256), 0,
                          st, p);
       return;

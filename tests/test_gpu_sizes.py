@@ -117,3 +117,29 @@ def test_transition_rows_c384(rows, inplace):
     with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16):
         got = mod.hip_apply(xg, out=xg, add_residual=True) if inplace else mod.hip_apply(xg)
     assert_bf16(got.cpu() - x if inplace else got, exp, f"transition rows={rows} inplace={inplace}")
+
+
+@pytest.mark.parametrize("n", [96, 111, 112, 160, 192, 193])
+@pytest.mark.parametrize("tf32", [False, True])
+@pytest.mark.parametrize("c", [64, 128])
+def test_staged_f32_sizes(n, tf32, c):
+    """The fp32 and three-part kernels with weights staged in LDS, one and two
+    rows per workgroup, on either side of their sizes, in place."""
+    say(f"[gpu] staged f32 n={n} tf32={tf32} c={c}")
+    z = torch.randn(n, n, c, generator=torch.Generator().manual_seed(n + c))
+    mask = token_pair_mask(n, 3)
+    att = seeded(TriangleAttention(c, 32, c // 32), n, 0.1)
+    mul = seeded(TriangleMultiplicationIncoming(c, c), n, 0.1)
+    ea = ref.triangle_attention(z, mask, params_of(att), c // 32)
+    em = ref.triangle_multiplication(z, mask, params_of(mul), outgoing=False)
+    old = torch.backends.cuda.matmul.allow_tf32
+    torch.backends.cuda.matmul.allow_tf32 = tf32
+    try:
+        with torch.no_grad():
+            for mod, exp, what in ((att, ea, "attention"), (mul, em, "multiplication")):
+                zd = z.to(DEV)
+                got = mod.to(DEV).hip_apply(zd, mask.to(DEV), out=zd, add_residual=True)
+                assert got.data_ptr() == zd.data_ptr()
+                assert_fp32(zd, z + exp, f"staged {what} n={n} tf32={tf32} c={c}")
+    finally:
+        torch.backends.cuda.matmul.allow_tf32 = old
