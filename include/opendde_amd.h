@@ -37,7 +37,7 @@ extern "C" {
  * operand as a bf16 pair hi + lo; hi*hi + hi*lo + lo*hi, f32 accumulation;
  * about 2^-16 of relative error per product): every projection, the
  * attention core, the outputs and the transition's GEMMs, and the triangle
- * contraction where Np is a multiple of 256 (true fp32 products otherwise;
+ * contraction where N rounded up to 128 is a multiple of 256 (true fp32 products otherwise;
  * the transition's pair-bias projection stays true fp32).  The f32 mode for
  * callers that allow reduced-precision products: the reference's kernel
  * slot and its linear layers take TF32 (2^-11) from

@@ -351,8 +351,8 @@ def triangle_multiplication(z: torch.Tensor, mask: Optional[torch.Tensor], *, ou
     f32 (it folds LN_out into that weight with a single bf16 rounding).
     fp32 arithmetic with ``torch.backends.cuda.matmul.allow_tf32`` set runs
     the products in three bf16 parts, as :func:`triangle_attention` does:
-    the projections and the output always, the contraction where Np is a
-    multiple of 256 (true fp32 products otherwise)."""
+    the projections and the output always, the contraction where N rounded
+    up to 128 is a multiple of 256 (true fp32 products otherwise)."""
     _require_gpu(z, mask)
     nbatch, z_sb, zs0, zs1 = _pair_strides(z, "z")
     n, c = z.shape[-3], z.shape[-1]
