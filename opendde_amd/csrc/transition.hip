@@ -800,9 +800,17 @@ struct TfStage {
 
 // kX3 (ODDE_F32X3): the products in three bf16 parts (rows and hidden
 // activations split once, weight fragments as they are read from LDS).
-template <typename ZT, int kC, int kW, bool kX3 = false>
+//
+// kSplit (true fp32 products): waves w and w + kW / 2 own the same 16 rows and
+// take one 16-unit half of every chunk each (lo or hi of GEMM2's fragments);
+// the sums meet in LDS at the end of a tile.  64 rows a workgroup then keep two
+// waves on every SIMD: one's LDS reads and silu run under the other's products
+// (C = 128, 16384 rows: 72 -> 67 us; the products alone take 43).
+template <typename ZT, int kC, int kW, bool kX3 = false, bool kSplit = false>
 __global__ __launch_bounds__(64 * kW) void transition_f32_pipe_kernel(TransitionArgs<ZT, float> a,
                                                                       int64_t ntiles) {
+  static_assert(!(kX3 && kSplit), "a 16-unit half is no whole bf16 fragment");
+  constexpr int kRW = kSplit ? kW / 2 : kW;  // waves with rows of their own
   constexpr int C = kC * 32, HID = 4 * C, NCB = C / 16, NCHUNK = HID / kTrHid;
   using MF = MulFrag<float, kX3>;
   constexpr int CPR = C / 4;                 // 16-byte chunks per W_a / W_b row
@@ -857,7 +865,7 @@ __global__ __launch_bounds__(64 * kW) void transition_f32_pipe_kernel(Transition
   const int key = r16 & 7;  // the swizzle key of every fragment row this lane reads
   int q = 0;
   for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-    const int64_t row = tile * (16 * kW) + 16 * w + r16;
+    const int64_t row = tile * (16 * kRW) + 16 * (w % kRW) + r16;
     const bool valid = row < a.rows;
     MF xf[kC];
     {
@@ -878,6 +886,30 @@ __global__ __launch_bounds__(64 * kW) void transition_f32_pipe_kernel(Transition
       barrier_nofence();
       if (q + 1 < Q) issue(q + 1);
       const TfStage<kC>& S = st[q & 1];
+      if constexpr (kSplit) {
+        const int hb = wu / kRW, rr = 16 * hb + r16;
+        f32x4 sa = {0.f, 0.f, 0.f, 0.f}, sb = sa, hh;
+#pragma unroll
+        for (int t = 0; t < kC; ++t) {
+          MF ma, mb;
+          ma.lo = S.wa[rr * CPR + ((8 * t + 2 * g) ^ key)];
+          ma.hi = S.wa[rr * CPR + ((8 * t + 2 * g + 1) ^ key)];
+          mb.lo = S.wb[rr * CPR + ((8 * t + 2 * g) ^ key)];
+          mb.hi = S.wb[rr * CPR + ((8 * t + 2 * g + 1) ^ key)];
+          mma(sa, ma, xf[t]);
+          mma(sb, mb, xf[t]);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) hh[e] = siluf_(sa[e]) * sb[e];
+#pragma unroll
+        for (int cb = 0; cb < NCB; ++cb) {
+          const f32x4 mo = S.wo[(16 * cb + r16) * 8 + ((4 * hb + g) ^ key)];
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            acc[cb] = __builtin_amdgcn_mfma_f32_16x16x4f32(mo[e], hh[e], acc[cb], 0, 0, 0);
+        }
+        continue;
+      }
       Frag<float> hf;
 #pragma unroll
       for (int hb = 0; hb < 2; ++hb) {
@@ -921,6 +953,24 @@ __global__ __launch_bounds__(64 * kW) void transition_f32_pipe_kernel(Transition
         }
         mma(acc[cb], mo, hm);
       }
+    }
+    if constexpr (kSplit) {
+      // the second half's sums through the stage of the tile's last chunk: the
+      // next chunk into it is issued after the barrier that opens the next
+      // chunk, which waits for these reads
+      f32x4* part = reinterpret_cast<f32x4*>(&st[(q - 1) & 1]) + (w % kRW) * (NCB * 64) + l;
+      static_assert(sizeof(st[0]) >= kRW * NCB * 64 * sizeof(f32x4), "the sums fit in a stage");
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      barrier_nofence();  // every wave is done with that chunk
+      if (wu >= kRW) {
+#pragma unroll
+        for (int cb = 0; cb < NCB; ++cb) part[cb * 64] = acc[cb];
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      barrier_nofence();
+      if (wu >= kRW) continue;
+#pragma unroll
+      for (int cb = 0; cb < NCB; ++cb) acc[cb] += part[cb * 64];
     }
     // epilogue: lane holds row r16 of the wave, channels 16 cb + 4g + e
 #pragma unroll
@@ -1431,25 +1481,41 @@ int run_transition_f32(const odde_transition_args* a, hipStream_t st) {
     p.wo = reinterpret_cast<const float*>(d);
   }
   LaunchScope ls(ODDE_K_TRANSITION, st);
-  // the staged form when its tiles fill the GPU and the weights can be
-  // staged by 16-byte direct loads
+  // The staged forms where the weights can be staged by 16-byte direct loads,
+  // from the row count on at which one tile of 64 rows through the whole hidden
+  // dimension is faster than the fragment form: that time hardly depends on
+  // the rows up to one tile per CU, the fragment form's does.  us, fragments /
+  // 4 waves / 8 waves in halves / 128 rows: C = 128 fp32, 5184 rows 49 / 70 / 62 /
+  // 108, 9216 78 / 70 / 63 / 109, 16384 124 / 72 / 67 / 112, 22500 148 / 139 / - /
+  // 116; three parts, 3136 40 / 37, 4096 47 / 37 / - / 46, 9216 77 / 40 / - / 47,
+  // 22500 147 / 72 / - / 52.  C = 64 fp32, 6400 22 / 24 / 21 / 33, 9216 25 / 23 / 23 /
+  // 34, 22500 - / 36 / 36; three parts, 4096 14 / 15, 5184 18 / 17, 9216 25 / 16.
   const bool aligned16 = ((reinterpret_cast<uintptr_t>(p.wa) | reinterpret_cast<uintptr_t>(p.wb) |
                            reinterpret_cast<uintptr_t>(p.wo)) & 15) == 0;
-  if (aligned16 && a->n_factor == 4 && (a->c == 64 || a->c == 128) && p.rows >= 256 * 64) {
-    if (p.rows >= 256 * 128) {  // 8 waves (128 rows) per workgroup, 2 per SIMD
-      const int64_t ntiles = (p.rows + 127) / 128;
-      const int g2 = (int)std::min<int64_t>(ntiles, a->c == 64 ? 2 * 256 : 256);
-      if (a->c == 64)
-        hipLaunchKernelGGL((transition_f32_pipe_kernel<float, 2, 8, kX3>), dim3(g2), dim3(512), 0, st, p, ntiles);
-      else
-        hipLaunchKernelGGL((transition_f32_pipe_kernel<float, 4, 8, kX3>), dim3(g2), dim3(512), 0, st, p, ntiles);
-    } else {  // 4 waves (64 rows) per workgroup: more workgroups for fewer rows
-      const int64_t ntiles = (p.rows + 63) / 64;
-      const int g2 = (int)std::min<int64_t>(ntiles, a->c == 64 ? 3 * 256 : 256);
-      if (a->c == 64)
-        hipLaunchKernelGGL((transition_f32_pipe_kernel<float, 2, 4, kX3>), dim3(g2), dim3(256), 0, st, p, ntiles);
-      else
-        hipLaunchKernelGGL((transition_f32_pipe_kernel<float, 4, 4, kX3>), dim3(g2), dim3(256), 0, st, p, ntiles);
+  const int64_t staged_rows = 256 * (kX3 ? (a->c == 128 ? 16 : 20) : (a->c == 128 ? 26 : 36));
+  if (aligned16 && a->n_factor == 4 && (a->c == 64 || a->c == 128) && p.rows >= staged_rows) {
+    auto launch = [&](auto kc_c, auto w_c, auto split_c, int cap) {
+      constexpr int kW = decltype(w_c)::value, kRows = decltype(split_c)::value ? 8 * kW : 16 * kW;
+      const int64_t ntiles = (p.rows + kRows - 1) / kRows;
+      hipLaunchKernelGGL((transition_f32_pipe_kernel<float, decltype(kc_c)::value, kW, kX3,
+                                                     decltype(split_c)::value>),
+                         dim3((unsigned)std::min<int64_t>(ntiles, cap)), dim3(64 * kW), 0, st, p,
+                         ntiles);
+    };
+    using K2 = std::integral_constant<int, 2>;
+    using K4 = std::integral_constant<int, 4>;
+    using W4 = std::integral_constant<int, 4>;
+    using W8 = std::integral_constant<int, 8>;
+    // C = 128 has one workgroup on a CU: 128 rows as soon as 64 leave a second round
+    if (p.rows >= 256 * 128 || (a->c == 128 && p.rows > 256 * 64)) {
+      if (a->c == 64) launch(K2{}, W8{}, std::false_type{}, 2 * 256);
+      else launch(K4{}, W8{}, std::false_type{}, 256);
+    } else if (a->c == 64) {
+      launch(K2{}, W4{}, std::false_type{}, 3 * 256);
+    } else if constexpr (kX3) {
+      launch(K4{}, W4{}, std::false_type{}, 256);
+    } else {
+      launch(K4{}, W8{}, std::true_type{}, 256);
     }
     return check_launch("transition (fp32)");
   }

@@ -143,3 +143,25 @@ def test_staged_f32_sizes(n, tf32, c):
                 assert_fp32(zd, z + exp, f"staged {what} n={n} tf32={tf32} c={c}")
     finally:
         torch.backends.cuda.matmul.allow_tf32 = old
+
+
+@pytest.mark.parametrize("rows", [4096, 6655, 6656, 9217, 16384, 16385])
+@pytest.mark.parametrize("tf32", [False, True])
+@pytest.mark.parametrize("c", [64, 128])
+def test_transition_f32_staged_rows(rows, tf32, c):
+    """The fp32 transition's forms on either side of their row counts: weight
+    fragments, 64 rows (in two hidden halves for true fp32) and 128 rows."""
+    from opendde_amd.pairformer import Transition
+    say(f"[gpu] transition f32 rows={rows} tf32={tf32} c={c}")
+    x = torch.randn(rows, c, generator=torch.Generator().manual_seed(rows + c))
+    mod = seeded(Transition(c, 4), 11, 0.07 * (128 / c) ** 0.5)
+    exp = ref.transition(x, params_of(mod))
+    old = torch.backends.cuda.matmul.allow_tf32
+    torch.backends.cuda.matmul.allow_tf32 = tf32
+    try:
+        xg = x.to(DEV)
+        with torch.no_grad():
+            mod.to(DEV).hip_apply(xg, out=xg, add_residual=True)
+        assert_fp32(xg, x + exp, f"transition f32 rows={rows} tf32={tf32} c={c}")
+    finally:
+        torch.backends.cuda.matmul.allow_tf32 = old
